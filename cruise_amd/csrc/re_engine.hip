@@ -34,9 +34,13 @@ namespace re {
 // its contents behind: nothing in it needs to start at zero, every byte a
 // pass reads is written earlier in the same pass).
 constexpr size_t kNoAllocScratchBytes = 64ull << 20;
+// Partial sums of the batched prefill's split GEMMs at most, in both entry
+// points alike, so both choose the same K ranges and compute the same bits.
+// (Unlimited, the plans of the 7B shape would take up to about 66 MiB.)
+constexpr size_t kPrefillPartBytes = 64ull << 20;
 }  // namespace re
 
-static __device__ __align__(256) uint8_t scratch[re::kNoAllocScratchBytes];
+static __device__ __align__(256) uint8_t scratch[re::kNoAllocScratchBytes + re::kPrefillPartBytes];
 
 namespace re {
 namespace {
@@ -1345,8 +1349,8 @@ namespace {
 // resident_epoch_prefill_batch).  Token i of the pass is (row, position);
 // a row's tokens are consecutive and start at position 0.
 // Scratch: the engine's own buffer, grown on demand, or (fixed != nullptr)
-// the caller's fixed buffer of fixed_bytes, in which case nothing is
-// allocated and a pass that does not fit returns -3.
+// the caller's fixed buffer of fixed_bytes and kPrefillPartBytes behind them,
+// in which case nothing is allocated and a pass that does not fit returns -3.
 int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector<int32_t>& gens,
                       const std::vector<std::vector<int64_t>>& prompts, const std::vector<int32_t>& tables,
                       uint8_t* fixed = nullptr, size_t fixed_bytes = 0) {
@@ -1392,8 +1396,18 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   const size_t o_mlp = take(M * I * T), o_rope = take((size_t)M * d.head_dim * sizeof(float));
   const size_t o_tok = take(8 * (size_t)M), o_pos = take(4 * (size_t)M), o_slot = take(4 * (size_t)M);
   const size_t o_tiles = take(sizeof(int4) * tiles.size()), o_blocks = take(4 * tables.size());
+  const size_t rows_bytes = off;
+  // K ranges of the qkv, o and down GEMMs (bf16); each one's partial sums are
+  // consumed before the next writes its own
+  auto plan_of = [&](int N, int K) { return fused_mlp && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
+  const GemmPlan qkv_plan = plan_of(d.qkv_rows(), d.hidden), o_plan = plan_of(d.hidden, d.q_dim()),
+                 down_plan = plan_of(d.hidden, d.intermediate);
+  size_t part_bytes = 0;
+  for (const auto& [p, n] : {std::pair{qkv_plan, d.qkv_rows()}, {o_plan, d.hidden}, {down_plan, d.hidden}})
+    if (p.splits > 1) part_bytes = std::max(part_bytes, (size_t)p.splits * M * n * sizeof(float));
+  const size_t o_part = fixed != nullptr ? fixed_bytes : take(part_bytes);
   if (fixed != nullptr) {
-    if (off > fixed_bytes) return -3;
+    if (rows_bytes > fixed_bytes) return -3;
   } else if (off > e.pf_bytes) {
     if (e.pf_mem) (void)hipFree(e.pf_mem);
     e.pf_mem = nullptr;
@@ -1433,8 +1447,9 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
     const long long cache_layer_elems = d.slots() * d.kv_dim();
     for (int l = 0; l < d.layers && err == hipSuccess; ++l) {
       const LayerOffsets& lo = e.layer_off[l];
+      float* part = reinterpret_cast<float*>(b + o_part);
       auto gemm = [&](size_t a_off, long long lda, size_t w_off, size_t bias_off, size_t out_off, long long ldo, int N,
-                      int K, int epi) {
+                      int K, int epi, GemmPlan plan = {4, 1}) {
         GemmArgs g{};
         g.A = b + a_off;
         g.W = e.weights + w_off;
@@ -1446,11 +1461,16 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
         g.lda = lda;
         g.ldw = K;
         g.ldo = ldo;
-        run(launch_gemm(g, epi, d.dtype_bytes, s));
+        if (plan.splits > 1) g.part = part;
+        run(launch_gemm(g, epi, d.dtype_bytes, s, plan));
       };
-      run(launch_prefill_rmsnorm(b + o_hidden, e.weights + lo.input_norm, b + o_xn, M, d.hidden, d.rms_eps,
-                                 d.dtype_bytes, s));
-      gemm(o_xn, d.hidden, lo.qkv_w, lo.qkv_b, o_qkv, d.qkv_rows(), d.qkv_rows(), d.hidden, kGemmStore);
+      // a split GEMM's partial sums are added by the launch that follows it
+      auto norm = [&](size_t w_off, const GemmPlan& before) {
+        run(launch_prefill_rmsnorm(b + o_hidden, e.weights + w_off, b + o_xn, M, d.hidden, d.rms_eps, d.dtype_bytes, part,
+                                   before.splits > 1 ? before.splits : 0, s));
+      };
+      norm(lo.input_norm, l > 0 ? down_plan : GemmPlan{4, 1});
+      gemm(o_xn, d.hidden, lo.qkv_w, lo.qkv_b, o_qkv, d.qkv_rows(), d.qkv_rows(), d.hidden, kGemmStore, qkv_plan);
       PrefillQkv qp{};
       qp.qkv = b + o_qkv;
       qp.rope = er.rope;
@@ -1463,6 +1483,9 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       qp.heads = d.heads;
       qp.kv_heads = d.kv_heads;
       qp.head_dim = d.head_dim;
+      qp.part = part;
+      qp.bias = e.weights + lo.qkv_b;
+      qp.parts = qkv_plan.splits > 1 ? qkv_plan.splits : 0;
       run(launch_prefill_qkv_post(qp, d.dtype_bytes, s));
       PrefillAttn at{};
       at.qkv = b + o_qkv;
@@ -1475,9 +1498,8 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       at.kv_heads = d.kv_heads;
       at.head_dim = d.head_dim;
       run(launch_prefill_attention(at, d, static_cast<int>(tiles.size()), s));
-      gemm(o_attn, d.q_dim(), lo.o_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.q_dim(), kGemmResidual);
-      run(launch_prefill_rmsnorm(b + o_hidden, e.weights + lo.post_norm, b + o_xn, M, d.hidden, d.rms_eps,
-                                 d.dtype_bytes, s));
+      gemm(o_attn, d.q_dim(), lo.o_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.q_dim(), kGemmResidual, o_plan);
+      norm(lo.post_norm, o_plan);
       if (fused_mlp) {
         GemmArgs g{};
         g.A = b + o_xn;
@@ -1496,7 +1518,8 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
         gemm(o_xn, d.hidden, lo.up_w, SIZE_MAX, o_up, d.intermediate, d.intermediate, d.hidden, kGemmStore);
         run(launch_prefill_swiglu(b + o_gate, b + o_up, b + o_mlp, (long long)M * d.intermediate, d.dtype_bytes, s));
       }
-      gemm(o_mlp, d.intermediate, lo.down_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.intermediate, kGemmResidual);
+      gemm(o_mlp, d.intermediate, lo.down_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.intermediate, kGemmResidual,
+           down_plan);  // the last layer's residual stream is not read
     }
     if (err != hipSuccess) return -2;
   }

@@ -288,6 +288,9 @@ struct PrefillQkv {            // RoPE in place + paged KV write
   void* value_cache;
   long long slots;
   int M, ld, heads, kv_heads, head_dim;
+  const float* part;           // parts > 0: the rows' partial sums [parts][M][q | k | v rows] (bf16)
+  const void* bias;            // T [q | k | v rows], with parts
+  int parts;
 };
 struct PrefillAttn {           // causal attention within each row's prompt
   const void* qkv;             // T [M, ld] after RoPE
@@ -299,7 +302,12 @@ struct PrefillAttn {           // causal attention within each row's prompt
 // Store: out = T(acc + bias); Residual: out = T(out + T(acc)); SwiGlu (bf16
 // only): W holds the gate rows and W2 the up rows, and out[m, n] =
 // T(T(silu(T(gate))) * T(up)) over N output columns.
-enum GemmEpilogue : int { kGemmStore = 0, kGemmResidual = 1, kGemmSwiGlu = 2 };
+// Part (bf16 only): the fp32 partial sums of K ranges, to part.
+enum GemmEpilogue : int { kGemmStore = 0, kGemmResidual = 1, kGemmSwiGlu = 2, kGemmPart = 3 };
+// Tile rows (64 mj) and K ranges of a bf16 GEMM (plan_gemm).
+struct GemmPlan {
+  int mj, splits;
+};
 struct GemmArgs {              // out[M,N] (epilogue) A[M,K] W[N,K]^T
   const void* A;
   const void* W;
@@ -308,14 +316,20 @@ struct GemmArgs {              // out[M,N] (epilogue) A[M,K] W[N,K]^T
   int M, N, K;
   long long lda, ldw, ldo;
   const void* W2;              // [N,K] up rows of the SwiGLU epilogue (W: the gate rows)
+  float* part;                 // not null: partial sums [ranges][M][N] instead of out (bf16)
 };
 hipError_t launch_prefill_embed(const PrefillRows& a, int dtype_bytes, hipStream_t stream);
-hipError_t launch_prefill_rmsnorm(const void* x, const void* w, void* y, int M, int H, float eps, int dtype_bytes,
-                                  hipStream_t stream);
+// parts > 0: x += the partial sums [parts][M][H] of a split GEMM first (bf16).
+hipError_t launch_prefill_rmsnorm(void* x, const void* w, void* y, int M, int H, float eps, int dtype_bytes,
+                                  const float* part, int parts, hipStream_t stream);
 hipError_t launch_prefill_swiglu(const void* gate, const void* up, void* out, long long n, int dtype_bytes,
                                  hipStream_t stream);
 hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStream_t stream);
-hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream);
+// The fastest tile and K ranges for a shape whose partial sums take at most
+// part_bytes; launch_gemm follows `plan` when a.part is set, else it picks the
+// tile itself and runs one K range.
+GemmPlan plan_gemm(int M, int N, int K, bool swiglu, size_t part_bytes);
+hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream, GemmPlan plan = {4, 1});
 // The MFMA attention serves bf16 models with head_dim 128 (64-query tiles).
 bool prefill_attention_mfma(const Dims& d);
 size_t prefill_attention_lds(const Dims& d, int max_keys);

@@ -5,13 +5,15 @@
 //   embed      token rows + per-token RoPE table
 //   rmsnorm    one workgroup per token
 //   GEMM       C[M,N] = A[M,K] W[N,K]^T, both operands K-contiguous.
-//              bf16: MFMA v_mfma_f32_16x16x32_bf16, 256x256 workgroup tiles
-//              (eight waves of 128x64), K in steps of 64 through two LDS
+//              bf16: MFMA v_mfma_f32_16x16x32_bf16, workgroup tiles of 256
+//              columns by 64 to 256 rows, K in steps of 64 through LDS
 //              stages filled by direct global -> LDS loads, fp32
 //              accumulation; epilogues "T(acc + bias)", the residual
 //              "T(h + T(acc))", and gate/up with SwiGLU in one GEMM (the
-//              tile's W rows half gate, half up).  fp32 models: an
-//              LDS-tiled FMA GEMM.
+//              tile's W rows half gate, half up); K split over workgroups
+//              where the tiles alone leave CUs idle, the partial sums added
+//              by the row kernel that follows.  fp32 models: an LDS-tiled
+//              FMA GEMM.
 //   qkv post   RoPE of q and k in place, K/V rows to their paged slots
 //   attention  causal within each row's prompt.  bf16, head_dim 128: MFMA
 //              for Q K^T and P V per (64-query tile, head), the bf16 scores of
@@ -42,6 +44,33 @@ __device__ __forceinline__ bf16x8_t lds_frag(const bf16_t* p) {
 // ---------------------------------------------------------------------------
 // Row kernels
 // ---------------------------------------------------------------------------
+// The partial sums of NV four-element vectors, added in range order; UNROLL
+// ranges' loads in flight at once (each is a round trip to memory that
+// another XCD wrote).
+template <int NV, int UNROLL>
+__device__ __forceinline__ void part_sums(const float* const (&p)[NV], size_t plane, int parts, re_f32x4 (&sum)[NV]) {
+  int r = 0;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) sum[v] = re_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto block = [&](auto n) {
+    re_f32x4 x[n][NV];
+#pragma unroll
+    for (int u = 0; u < n; ++u)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) x[u][v] = *reinterpret_cast<const re_f32x4*>(p[v] + (r + u) * plane);
+#pragma unroll
+    for (int u = 0; u < n; ++u)
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[v][e] += x[u][v][e];
+    r += n;
+  };
+  while (r + UNROLL <= parts) block(std::integral_constant<int, UNROLL>{});
+  while (r + 2 <= parts) block(std::integral_constant<int, 2>{});
+  if (r < parts) block(std::integral_constant<int, 1>{});
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_pf_embed(PrefillRows a) {
   const int m = blockIdx.x, tid = threadIdx.x;
@@ -60,30 +89,61 @@ __global__ void __launch_bounds__(256) k_pf_embed(PrefillRows a) {
 }
 
 // RMSNorm (batched_decoder_step.py:224-229): fp32 mean of squares, rsqrt,
-// cast to T, T x T product with the weight.
-template <typename T>
-__global__ void __launch_bounds__(256) k_pf_rmsnorm(const void* x, const void* w, void* y, int H, float eps) {
-  __shared__ float red[4];
+// cast to T, T x T product with the weight.  One workgroup per token, its row
+// in registers (H <= 4,096).
+//
+// PART: the residual add of the preceding split GEMM comes first, h =
+// T(h + T(p_0 + p_1 + ...)) over its fp32 partials [parts][M][H] in range
+// order (the residual epilogue's roundings), written back to x.
+// PART runs one 8-element vector per thread (512 threads), so all of a row's
+// partials are on their way in two or three round trips.
+constexpr int kNormRow = 4096;
+template <typename T, bool PART>
+__global__ void __launch_bounds__(PART ? 512 : 256) k_pf_rmsnorm(void* x, const void* w, void* y, int H, float eps,
+                                                                 const float* part, int parts) {
+  constexpr int kThreads = PART ? 512 : 256, kNormVecs = kNormRow / 8 / kThreads;
+  __shared__ float red[kThreads / 64];
   const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const T* xr = static_cast<const T*>(x) + (size_t)m * H;
+  T* xr = static_cast<T*>(x) + (size_t)m * H;
   const T* wr = static_cast<const T*>(w);
   T* yr = static_cast<T*>(y) + (size_t)m * H;
+  const size_t plane = (size_t)gridDim.x * H;
+  Vec8<T> v[kNormVecs];
   float s = 0.f;
-  for (int c = tid; c < H / 8; c += 256) {
-    const Vec8<T> v = Vec8<T>::load_cached(xr + c * 8);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s = fmaf(v.get(e), v.get(e), s);
+  for (int i = 0; i < kNormVecs; ++i) {
+    const int c = tid + kThreads * i;
+    if (c * 8 >= H) continue;
+    v[i] = Vec8<T>::load_cached(xr + c * 8);
+    if constexpr (PART) {
+      const float* p0 = part + (size_t)m * H + c * 8;
+      const float* const p[2] = {p0, p0 + 4};
+      re_f32x4 ps[2];
+      part_sums<2, 7>(p, plane, parts, ps);
+      float nh[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nh[e] = Elt<T>::r(v[i].get(e) + Elt<T>::r(ps[e >> 2][e & 3]));
+      v[i] = Vec8<T>::from_floats(nh);
+      *reinterpret_cast<Vec8<T>*>(xr + c * 8) = v[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = fmaf(v[i].get(e), v[i].get(e), s);
   }
   s = wave_sum(s);
   if (lane == 0) red[wave] = s;
   __syncthreads();
-  const float rs = rsqrtf((red[0] + red[1] + red[2] + red[3]) / static_cast<float>(H) + eps);
-  for (int c = tid; c < H / 8; c += 256) {
-    const Vec8<T> v = Vec8<T>::load_cached(xr + c * 8);
+  float total = red[0];
+#pragma unroll
+  for (int i = 1; i < kThreads / 64; ++i) total += red[i];
+  const float rs = rsqrtf(total / static_cast<float>(H) + eps);
+#pragma unroll
+  for (int i = 0; i < kNormVecs; ++i) {
+    const int c = tid + kThreads * i;
+    if (c * 8 >= H) continue;
     const Vec8<T> g = Vec8<T>::load_cached(wr + c * 8);
     float out[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = Elt<T>::r(Elt<T>::r(v.get(e) * rs) * g.get(e));
+    for (int e = 0; e < 8; ++e) out[e] = Elt<T>::r(Elt<T>::r(v[i].get(e) * rs) * g.get(e));
     *reinterpret_cast<Vec8<T>*>(yr + c * 8) = Vec8<T>::from_floats(out);
   }
 }
@@ -128,8 +188,12 @@ __device__ __forceinline__ void store8<float>(float* p, const Vec8<float>& v) {
 // One workgroup per token; a thread takes 8 consecutive pair indices j of one
 // head (16-byte accesses of both halves, the RoPE table's 8 cos/sin pairs),
 // head_dim a multiple of 16.
-template <typename T>
-__global__ void __launch_bounds__(256) k_pf_qkv_post(PrefillQkv a) {
+//
+// PART: the rows come from the split GEMM's fp32 partials instead, T(p_0 +
+// p_1 + ... + bias) (the store epilogue's rounding), v written to the rows too.
+// Its workgroups have a thread per vector pair where 512 threads allow it.
+template <typename T, bool PART>
+__global__ void __launch_bounds__(PART ? 512 : 256) k_pf_qkv_post(PrefillQkv a) {
   const int m = blockIdx.x;
   const int half = a.head_dim / 2, hv = half / 8;
   const int nq = a.heads, nkv = a.kv_heads;
@@ -140,7 +204,27 @@ __global__ void __launch_bounds__(256) k_pf_qkv_post(PrefillQkv a) {
   for (int idx = threadIdx.x; idx < (nq + 2 * nkv) * hv; idx += blockDim.x) {
     const int hg = idx / hv, j = (idx - hg * hv) * 8;
     T* p = row + (size_t)hg * a.head_dim;
-    Vec8<T> va = Vec8<T>::load_cached(p + j), vb = Vec8<T>::load_cached(p + j + half);
+    Vec8<T> va, vb;
+    if constexpr (PART) {
+      const int n0 = hg * a.head_dim + j, np = (nq + 2 * nkv) * a.head_dim;
+      const float* pp = a.part + (size_t)m * np + n0;
+      const float* const ps[4] = {pp, pp + 4, pp + half, pp + half + 4};
+      re_f32x4 sum[4];
+      part_sums<4, 5>(ps, (size_t)a.M * np, a.parts, sum);
+      float sa[8], sb[8];
+      const T* bias = static_cast<const T*>(a.bias) + n0;
+      const Vec8<T> ba = Vec8<T>::load_cached(bias), bb = Vec8<T>::load_cached(bias + half);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        sa[e] = Elt<T>::r(sum[e >> 2][e & 3] + ba.get(e));
+        sb[e] = Elt<T>::r(sum[2 + (e >> 2)][e & 3] + bb.get(e));
+      }
+      va = Vec8<T>::from_floats(sa);
+      vb = Vec8<T>::from_floats(sb);
+    } else {
+      va = Vec8<T>::load_cached(p + j);
+      vb = Vec8<T>::load_cached(p + j + half);
+    }
     if (hg < nq + nkv) {
       float oa[8], ob[8];
 #pragma unroll
@@ -152,6 +236,8 @@ __global__ void __launch_bounds__(256) k_pf_qkv_post(PrefillQkv a) {
       }
       va = Vec8<T>::from_floats(oa);
       vb = Vec8<T>::from_floats(ob);
+    }
+    if (PART || hg < nq + nkv) {
       store8<T>(p + j, va);
       store8<T>(p + j + half, vb);
     }
@@ -168,45 +254,56 @@ __global__ void __launch_bounds__(256) k_pf_qkv_post(PrefillQkv a) {
 // ---------------------------------------------------------------------------
 // GEMMs
 // ---------------------------------------------------------------------------
-// bf16: one 256 x 256 output tile per workgroup of 8 waves, K in steps of 64.
+// bf16: one 64 MJ x 256 output tile (MJ = 1 .. 4) per workgroup of 8 waves, K
+// in steps of 64, over all of K or over one of nS ranges of it.
 //
 // Operands reach LDS by direct global -> LDS loads (global_load_lds_dwordx4,
-// 16 bytes per lane, no register staging) into two stages of 64 KB: W tile
-// rows 0..255, then A tile rows 256..511, 128 bytes (one K step) per row.
+// 16 bytes per lane, no register staging) into ST stages of 32 + 8 MJ KB: W
+// tile rows 0..255, then the A tile's rows, 128 bytes (one K step) per row.
 // Chunk c (16 bytes) of row r sits in slot c ^ gemm_swz(r), so the fragment
 // reads below hit distinct banks for 8 and for 16 consecutive rows.  The
 // products run as C^T = W A^T on v_mfma_f32_16x16x32_bf16: wave (wn, wm) owns
-// n 128 x m 64 (8 x 4 tiles of 16 x 16), and a lane's accumulator holds four
+// n 128 x m 16 MJ (8 x MJ tiles of 16 x 16), and a lane's accumulator holds four
 // consecutive output columns of one row.  A stage is two sub-steps of K = 32;
-// each sub-step's 12 fragments are read under the previous sub-step's 32
-// products, one read per two products.  The stage's one barrier sits between
-// its sub-steps: before it each wave waits for its own loads of stage kt + 1
-// and its reads of stage kt, so after it stage kt + 1 is complete in LDS and
-// stage kt's buffer is free.  The loads of stage kt + 2 go out during the
-// second sub-step (waves 0-3 at its start, waves 4-7 after 12 of their 32
-// products, so the two waves of a SIMD do not stall on them together), and
-// stage kt + 1's first fragments are read under the second sub-step's
-// products, so no wave waits on LDS at a stage boundary.  The
-// epilogue rounds the tile to bf16 in LDS (rows padded to 264 elements) and
-// writes it as row-contiguous 16-byte vectors: "T(acc + bias)" (qkv), or the
-// residual "T(h + T(acc))".
+// each sub-step's 8 + MJ fragments are read under the previous sub-step's 8 MJ
+// products.  The stage's one barrier sits between its sub-steps: before it
+// each wave waits for its own loads of stage kt + 1 and its reads of stage
+// kt, so after it stage kt + 1 is complete in LDS and stage kt's buffer is
+// free.  The loads of stage kt + ST go out during the second sub-step (waves
+// 0-3 at its start, waves 4-7 after 3 of their 8 row blocks, so the two waves
+// of a SIMD do not stall on them together), and stage kt + 1's first
+// fragments are read under the second sub-step's products, so no wave waits
+// on LDS at a stage boundary.  The epilogue rounds the tile to bf16 in LDS
+// (rows padded to 264 elements) and writes it as row-contiguous 16-byte
+// vectors: "T(acc + bias)" (qkv), or the residual "T(h + T(acc))"; a K range's
+// sums leave as fp32 from the accumulators, for the next launch to add.
+//
+// What bounds it: 256-row tiles the loop that feeds the matrix cores from LDS
+// (about 1.2 us a stage with every CU busy, 0.5 of the bf16 peak).  A call of
+// few rows has few tiles (14-18 for the 3,584- and 4,608-column products of
+// up to 256 rows on 256 CUs) and is bound by that serial loop, not by memory;
+// lower tiles shorten a stage (0.66 us at 64 rows, where three stages fit LDS
+// and 80 KB of loads stay in flight), K ranges the number of stages.
 //
 // Workgroups are dispatched round-robin over the 8 XCDs; workgroup b runs
-// tile t = (b % 8) * ceil(T / 8) + b / 8 of a grouped order (4 M tiles by
-// every N tile), so the 32 tiles an XCD runs at once share 4 A and 8 W row
-// blocks in its L2.
+// tile t = (b % 8) * ceil(T / 8) + b / 8 of an order with the K ranges
+// outermost and the tiles of a range grouped (4 M tiles by every N tile), so
+// the 32 tiles an XCD runs at once share 4 A and 8 W row blocks in its L2,
+// and the tiles of a K range share its columns of A.
 //
 // Requirements (checked by launch_gemm): K % 64 == 0, N % 8 == 0, lda, ldw
 // and ldo multiples of 8 elements, 16-byte aligned operands.
-constexpr int kGm = 256, kGn = 256, kGk = 64;
+constexpr int kGn = 256, kGk = 64;
 constexpr int kGrowBytes = kGk * 2;                   // one K step of one row
-constexpr int kGstage = (kGm + kGn) * kGrowBytes;     // 64 KB
 constexpr int kGwaves = 8, kGthreads = kGwaves * 64;
-constexpr int kGdmaRows = (kGm + kGn) / kGwaves;      // rows each wave loads per stage
-constexpr int kGdmaInsts = kGdmaRows / 8;             // 8 rows (1 KB) per instruction
 constexpr int kGoutLd = kGn + 8;                      // epilogue row stride (elements)
-constexpr int kGsmem = kGm * kGoutLd * 2 > 2 * kGstage ? kGm * kGoutLd * 2 : 2 * kGstage;
 constexpr int kGgroupM = 4;
+constexpr int gemm_tile_m(int mj) { return 64 * mj; }
+constexpr int gemm_stage_bytes(int mj) { return (kGn + gemm_tile_m(mj)) * kGrowBytes; }
+constexpr int gemm_stages(int mj) { return mj <= 2 ? 3 : 2; }
+constexpr int gemm_lds_bytes(int mj, int st) {
+  return std::max(gemm_tile_m(mj) * kGoutLd * 2, st * gemm_stage_bytes(mj));
+}
 
 typedef const __attribute__((address_space(1))) void* gemm_gptr;
 typedef __attribute__((address_space(3))) void* gemm_lptr;
@@ -216,146 +313,226 @@ __device__ __forceinline__ int gemm_swz(int r) { return (r & 7) ^ ((r >> 3) & 1)
 // s_waitcnt immediate: vmcnt <= vm (6 bits), lgkmcnt 0, expcnt untouched.
 constexpr int gemm_wait_vm(int vm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4); }
 
-// End of a stage: this wave's loads and LDS reads are done, then the barrier.
-// The empty asm statements keep the compiler from moving memory accesses
-// across; the wait is a real instruction the wait-count pass accounts for.
+// End of a stage: this wave's LDS reads and all but the last VM of its loads
+// are done, then the barrier.  The empty asm statements keep the compiler
+// from moving memory accesses across; the wait is a real instruction the
+// wait-count pass accounts for.
+template <int VM = 0>
 __device__ __forceinline__ void gemm_stage_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(gemm_wait_vm(0));
+  __builtin_amdgcn_s_waitcnt(gemm_wait_vm(VM));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ void gemm_tile_of(int b, int nM, int nN, int& mt, int& nt) {
-  const int total = nM * nN, x = b & 7, local = b >> 3, q = total >> 3, r = total & 7;
-  const int t = x < r ? x * (q + 1) + local : r * (q + 1) + (x - r) * q + local;
+// Tile and K range of workgroup b (see above): K ranges outermost.
+__device__ __forceinline__ void gemm_tile_of(int b, int nM, int nN, int nS, int& mt, int& nt, int& ks) {
+  const int tiles = nM * nN, total = tiles * nS, x = b & 7, local = b >> 3, q = total >> 3, r = total & 7;
+  int t = x < r ? x * (q + 1) + local : r * (q + 1) + (x - r) * q + local;
+  ks = t / tiles;
+  t -= ks * tiles;
   const int per_group = kGgroupM * nN, g = t / per_group, first = g * kGgroupM;
   const int gm = min(kGgroupM, nM - first), w = t - g * per_group;
   mt = first + w % gm;
   nt = w / gm;
 }
 
-template <int EPI>
-__global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, int nN) {
+// Fragments of the next stage read before product p of the second sub-step:
+// one per two products where that covers them, else spread over the first 7/8
+// of the products.
+constexpr int gemm_reads_by(int mj, int p) {
+  const int frags = 8 + mj, prods = 8 * mj, span = prods - prods / 8;
+  const int n = 2 * frags <= prods ? p / 2 : (p * frags + span - 1) / span;
+  return n < frags ? n : frags;
+}
+
+template <int EPI, int MJ, int ST>
+__global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, int nN, int nS) {
   extern __shared__ __align__(16) unsigned char gsm[];
+  constexpr int kTm = gemm_tile_m(MJ), kStage = gemm_stage_bytes(MJ);
+  constexpr int kInsts = 4 + MJ;  // 1 KB loads (8 rows) of each wave and stage
   // wave-uniform, so the load base lives in SGPRs (32-bit per-lane offsets)
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
-  int mt, nt;
-  gemm_tile_of(blockIdx.x, nM, nN, mt, nt);
-  // The SwiGLU epilogue's tile covers 128 output columns: W tile rows 0..127
-  // are their gate rows, rows 128..255 their up rows.
+  int mt, nt, ks;
+  gemm_tile_of(blockIdx.x, nM, nN, nS, mt, nt, ks);
+  // The SwiGLU tile covers 128 output columns: W tile rows 0..127 are their
+  // gate rows, rows 128..255 their up rows.
+  constexpr bool kPart = EPI == kGemmPart;
   constexpr bool kSwiGlu = EPI == kGemmSwiGlu;
   constexpr int kTileN = kSwiGlu ? kGn / 2 : kGn;
-  const int m0 = mt * kGm, n0 = nt * kTileN;
-  // Loads: waves 0-3 bring W rows 0..255, waves 4-7 A rows 0..255.  Rows past
-  // M or N read a valid row (clamped) whose results are never stored.
-  const int row0 = wave * kGdmaRows;
-  const bool loads_w = row0 < kGn;
-  const void* wsrc = kSwiGlu && row0 >= kTileN ? a.W2 : a.W;
-  const char* gbase = loads_w ? static_cast<const char*>(wsrc) + (size_t)n0 * a.ldw * 2
-                              : static_cast<const char*>(a.A) + (size_t)m0 * a.lda * 2;
-  const long long ld = loads_w ? a.ldw : a.lda;
-  const int rows_left = loads_w ? a.N - n0 : a.M - m0;
-  uint32_t goff[kGdmaInsts];
+  const int m0 = mt * kTm, n0 = nt * kTileN;
+  // K steps of this workgroup: range ks of nS nearly equal ones
+  const int steps = a.K / kGk;
+  const int k_begin = kPart ? static_cast<int>((long long)ks * steps / nS) : 0;
+  const int nk = (kPart ? static_cast<int>((long long)(ks + 1) * steps / nS) : steps) - k_begin;
+  // Loads.  256-row tiles: waves 0-3 bring W rows 0..255, waves 4-7 A rows
+  // 0..255.  Smaller ones: every wave 32 W rows (4 loads) and 8 MJ A rows.
+  // Rows past M or N read a valid row (clamped) whose results are never stored.
+  constexpr bool kSplitLoads = MJ == 4;
+  const char* wbase;
+  const char* abase = static_cast<const char*>(a.A) + (size_t)m0 * a.lda * 2 + (size_t)k_begin * kGrowBytes;
+  uint32_t goff[kInsts];
+  int lrow[2];  // tile row of the wave's first W (or only) load and of its first A load
+  if constexpr (kSplitLoads) {
+    const int row0 = wave * 64;
+    const bool loads_w = row0 < kGn;
+    const void* wsrc = kSwiGlu && row0 >= kTileN ? a.W2 : a.W;
+    wbase = loads_w ? static_cast<const char*>(wsrc) + (size_t)n0 * a.ldw * 2 + (size_t)k_begin * kGrowBytes : abase;
+    const long long ld = loads_w ? a.ldw : a.lda;
+    const int rows_left = loads_w ? a.N - n0 : a.M - m0;
 #pragma unroll
-  for (int i = 0; i < kGdmaInsts; ++i) {
-    // lane l of instruction i writes slot l % 8 of row row0 + 8 i + l / 8
-    const int row = row0 + i * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ gemm_swz(row);
-    const int local = loads_w ? row % kTileN : row & 255;  // the row within its source matrix
-    goff[i] = static_cast<uint32_t>(min(local, rows_left - 1) * ld * 2 + chunk * 16);
+    for (int i = 0; i < kInsts; ++i) {
+      // lane l of instruction i writes slot l % 8 of row row0 + 8 i + l / 8
+      const int row = row0 + i * 8 + (lane >> 3);
+      const int chunk = (lane & 7) ^ gemm_swz(row);
+      const int local = loads_w ? row % kTileN : row & 255;  // the row within its source matrix
+      goff[i] = static_cast<uint32_t>(min(local, rows_left - 1) * ld * 2 + chunk * 16);
+    }
+    lrow[0] = lrow[1] = row0;
+  } else {
+    lrow[0] = wave * 32;
+    lrow[1] = kGn + wave * 8 * MJ;
+    const void* wsrc = kSwiGlu && lrow[0] >= kTileN ? a.W2 : a.W;
+    wbase = static_cast<const char*>(wsrc) + (size_t)n0 * a.ldw * 2 + (size_t)k_begin * kGrowBytes;
+#pragma unroll
+    for (int i = 0; i < kInsts; ++i) {
+      const int row = (i < 4 ? lrow[0] + i * 8 : lrow[1] + (i - 4) * 8) + (lane >> 3);
+      const int chunk = (lane & 7) ^ gemm_swz(row);
+      goff[i] = i < 4 ? static_cast<uint32_t>(min(row % kTileN, a.N - n0 - 1) * a.ldw * 2 + chunk * 16)
+                      : static_cast<uint32_t>(min(row - kGn, a.M - m0 - 1) * a.lda * 2 + chunk * 16);
+    }
   }
-  const int nk = a.K / kGk;
-  auto issue = [&](int kt) {  // stages past the end re-read the last one (clamped, never used)
-    const char* g = gbase + (size_t)min(kt, nk - 1) * kGrowBytes;
-    unsigned char* l = gsm + (kt & 1) * kGstage + row0 * kGrowBytes;
+  auto issue = [&](int kt, int buf) {
+    const size_t kb = (size_t)kt * kGrowBytes;
+    unsigned char* l = gsm + buf * kStage;
+    if constexpr (kSplitLoads) {
 #pragma unroll
-    for (int i = 0; i < kGdmaInsts; ++i)
-      __builtin_amdgcn_global_load_lds((gemm_gptr)(g + goff[i]), (gemm_lptr)(l + i * 1024), 16, 0, 0);
+      for (int i = 0; i < kInsts; ++i)
+        __builtin_amdgcn_global_load_lds((gemm_gptr)(wbase + kb + goff[i]),
+                                         (gemm_lptr)(l + lrow[0] * kGrowBytes + i * 1024), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_global_load_lds((gemm_gptr)(wbase + kb + goff[i]),
+                                         (gemm_lptr)(l + lrow[0] * kGrowBytes + i * 1024), 16, 0, 0);
+#pragma unroll
+      for (int i = 4; i < kInsts; ++i)
+        __builtin_amdgcn_global_load_lds((gemm_gptr)(abase + kb + goff[i]),
+                                         (gemm_lptr)(l + lrow[1] * kGrowBytes + (i - 4) * 1024), 16, 0, 0);
+    }
   };
   const int wn = wave & 1, wm = wave >> 1;
-  f32x4_t acc[8][4];
+  f32x4_t acc[8][MJ];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < MJ; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
   // lane l supplies row l % 16 of a 16-row operand tile, K elements
   // 8 (l / 16) ..+8 of the 32-wide sub-step
   const int fr = lane & 15, fq = lane >> 4;
-  auto frag = [&](int st, int row, int ks) -> bf16x8_t {
-    const int c = (4 * ks + fq) ^ gemm_swz(row);
-    return lds_frag(reinterpret_cast<const bf16_t*>(gsm + st * kGstage + row * kGrowBytes + c * 16));
+  // (16-row tiles start at multiples of 16, so their row's swizzle is fr's)
+  const int frag_off[2] = {fr * kGrowBytes + ((fq ^ gemm_swz(fr)) * 16), fr * kGrowBytes + (((4 + fq) ^ gemm_swz(fr)) * 16)};
+  auto frag = [&](int st, int row0, int ks2) -> bf16x8_t {
+    return lds_frag(reinterpret_cast<const bf16_t*>(gsm + st * kStage + row0 * kGrowBytes + frag_off[ks2]));
   };
-  // fragment sets: [set][0..7] W rows (n), [set][8..11] A rows (m)
-  bf16x8_t f[2][12];
-  auto read_set = [&](int set, int st, int ks) {
+  // fragment sets: [set][0..7] W rows (n), [set][8..] A rows (m)
+  constexpr int kFrags = 8 + MJ, kProds = 8 * MJ;
+  bf16x8_t f[2][kFrags];
+  auto read_frag = [&](int set, int idx, int st, int ks2) {
+    f[set][idx] = idx < 8 ? frag(st, wn * 128 + idx * 16, ks2) : frag(st, kGn + wm * 16 * MJ + (idx - 8) * 16, ks2);
+  };
+  auto read_set = [&](int set, int st, int ks2) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) f[set][i] = frag(st, wn * 128 + i * 16 + fr, ks);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f[set][8 + j] = frag(st, kGn + wm * 64 + j * 16 + fr, ks);
+    for (int i = 0; i < kFrags; ++i) read_frag(set, i, st, ks2);
   };
   auto products = [&](int set) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < MJ; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[set][i], f[set][8 + j], acc[i][j], 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < 12; ++r) {  // one fragment read per two products
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    for (int r = 0; r < kFrags; ++r) {  // fragment reads spread over the products
+      __builtin_amdgcn_sched_group_barrier(0x008, kProds / kFrags > 0 ? kProds / kFrags : 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  issue(0);
-  issue(1);
-  __builtin_amdgcn_s_waitcnt(gemm_wait_vm(kGdmaInsts));  // this wave's stage 0
+  // Stages 0..ST-1 go out at once.  With 256-row tiles and one K range a
+  // stage past the end re-reads the last one (never used): without the branch
+  // around the loads the loop is 0.6 % faster, and K is long.  Elsewhere
+  // (ranges of a few stages) a stage that does not exist is not read.
+  constexpr bool kAlways = MJ == 4 && !kPart;
+  const int first = kAlways ? ST : min(ST, nk);
+  for (int s = 0; s < first; ++s) issue(kAlways ? min(s, nk - 1) : s, s);
+  if (first == ST)
+    __builtin_amdgcn_s_waitcnt(gemm_wait_vm((ST - 1) * kInsts));  // this wave's stage 0
+  else
+    __builtin_amdgcn_s_waitcnt(gemm_wait_vm(0));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   read_set(0, 0, 0);
   __builtin_amdgcn_sched_barrier(0);
+  int ring = 0;
   for (int kt = 0; kt < nk; ++kt) {
-    const int st = kt & 1;
+    const int st = ST == 2 ? kt & 1 : ring, nst = ST == 2 ? st ^ 1 : ring + 1 == ST ? 0 : ring + 1;
     read_set(1, st, 1);
     products(0);
-    gemm_stage_barrier();  // stage kt + 1 complete, stage kt's buffer free
-    // Second sub-step, in a fixed order: the 32 products row block by row
-    // block, the next stage's 12 first fragments one per two products (past
-    // the last stage: a buffer in flight, never used), and the loads of
-    // stage kt + 2.  The two waves of a SIMD (w and w + 4) issue their loads
-    // apart: an issuing wave waits while the memory pipeline takes its
-    // eight 1 KB requests, and meanwhile the other wave's products run.
+    // stage kt + 1 complete (stages kt + 2 .. kt + ST - 1 may be in flight),
+    // stage kt's buffer free
+    if (ST > 2 && kt + ST - 1 < nk)
+      gemm_stage_barrier<(ST - 2) * kInsts>();
+    else
+      gemm_stage_barrier();
+    const bool more = kAlways || kt + ST < nk;
+    const int next = kAlways ? min(kt + ST, nk - 1) : kt + ST;
+    // Second sub-step, in a fixed order: the products row block by row block,
+    // the next stage's first fragments between them (past the last stage: a
+    // stale buffer, never used), and the loads of stage kt + ST.  The two
+    // waves of a SIMD (w and w + 4) issue their loads apart: an issuing wave
+    // waits while the memory pipeline takes its 1 KB requests, and meanwhile
+    // the other wave's products run.
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (i == 0 && wave < 4) issue(kt + 2);
-      if (i == 3 && wave >= 4) issue(kt + 2);
+      if (i == 0 && wave < 4 && more) issue(next, st);
+      if (i == 3 && wave >= 4 && more) issue(next, st);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MJ; ++j) {
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][i], f[1][8 + j], acc[i][j], 0, 0, 0);
-        if (i < 6 && (j & 1)) {
-          const int idx = 2 * i + (j >> 1);
-          f[0][idx] = idx < 8 ? frag(st ^ 1, wn * 128 + idx * 16 + fr, 0)
-                              : frag(st ^ 1, kGn + wm * 64 + (idx - 8) * 16 + fr, 0);
-        }
+#pragma unroll
+        for (int r = gemm_reads_by(MJ, i * MJ + j); r < gemm_reads_by(MJ, i * MJ + j + 1); ++r) read_frag(0, r, nst, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    ring = nst;
   }
-  gemm_stage_barrier();
   // acc[i][j] value v of lane l: n = 16 i + 4 (l / 16) + v, m = 16 j + l % 16
   // within the wave's block
+  if constexpr (kPart) {
+    // fp32 partial sums [nS][M][N], four consecutive columns per lane
+#pragma unroll
+    for (int j = 0; j < MJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int m = m0 + wm * 16 * MJ + j * 16 + fr, n = n0 + wn * 128 + i * 16 + 4 * fq;
+        if (m < a.M && n < a.N)
+          *reinterpret_cast<f32x4_t*>(a.part + ((size_t)ks * a.M + m) * a.N + n) = acc[i][j];
+      }
+    return;
+  }
+  gemm_stage_barrier();
   bf16_t* T = reinterpret_cast<bf16_t*>(gsm);
   const bf16_t* bias = static_cast<const bf16_t*>(a.bias);
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < MJ; ++j)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int ml = wm * 64 + j * 16 + fr, nl = wn * 128 + i * 16 + 4 * fq;
+      const int ml = wm * 16 * MJ + j * 16 + fr, nl = wn * 128 + i * 16 + 4 * fq;
       float y[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = acc[i][j][e];
@@ -377,7 +554,7 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
     // column n0 + c: silu as the decode step computes it, rounded, then the
     // rounded product
 #pragma unroll 4
-    for (int idx = tid; idx < kGm * kTileN / 8; idx += kGthreads) {
+    for (int idx = tid; idx < kTm * kTileN / 8; idx += kGthreads) {
       const int r = idx / (kTileN / 8), c = idx % (kTileN / 8);
       const int m = m0 + r, n = n0 + c * 8;
       if (m >= a.M || n >= a.N) continue;
@@ -395,7 +572,7 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
     return;
   }
 #pragma unroll 4
-  for (int idx = tid; idx < kGm * kGn / 8; idx += kGthreads) {
+  for (int idx = tid; idx < kTm * kGn / 8; idx += kGthreads) {
     const int r = idx / (kGn / 8), c = idx % (kGn / 8);
     const int m = m0 + r, n = n0 + c * 8;
     if (m >= a.M || n >= a.N) continue;
@@ -808,13 +985,16 @@ hipError_t launch_prefill_embed(const PrefillRows& a, int dtype_bytes, hipStream
   return hipGetLastError();
 }
 
-hipError_t launch_prefill_rmsnorm(const void* x, const void* w, void* y, int M, int H, float eps, int dtype_bytes,
-                                  hipStream_t stream) {
+hipError_t launch_prefill_rmsnorm(void* x, const void* w, void* y, int M, int H, float eps, int dtype_bytes,
+                                  const float* part, int parts, hipStream_t stream) {
   if (M <= 0) return hipSuccess;
-  if (dtype_bytes == 2)
-    k_pf_rmsnorm<bf16_t><<<M, 256, 0, stream>>>(x, w, y, H, eps);
+  if (H % 8 != 0 || H > kNormRow || (parts > 0 && dtype_bytes != 2)) return hipErrorInvalidValue;
+  if (parts > 0)
+    k_pf_rmsnorm<bf16_t, true><<<M, 512, 0, stream>>>(x, w, y, H, eps, part, parts);
+  else if (dtype_bytes == 2)
+    k_pf_rmsnorm<bf16_t, false><<<M, 256, 0, stream>>>(x, w, y, H, eps, nullptr, 0);
   else
-    k_pf_rmsnorm<float><<<M, 256, 0, stream>>>(x, w, y, H, eps);
+    k_pf_rmsnorm<float, false><<<M, 256, 0, stream>>>(x, w, y, H, eps, nullptr, 0);
   return hipGetLastError();
 }
 
@@ -833,14 +1013,74 @@ hipError_t launch_prefill_swiglu(const void* gate, const void* up, void* out, lo
 hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStream_t stream) {
   if (a.M <= 0) return hipSuccess;
   if (a.head_dim % 16 != 0 || a.ld % 8 != 0) return hipErrorInvalidValue;
-  if (dtype_bytes == 2)
-    k_pf_qkv_post<bf16_t><<<a.M, 256, 0, stream>>>(a);
-  else
-    k_pf_qkv_post<float><<<a.M, 256, 0, stream>>>(a);
+  if (a.parts > 0) {
+    if (dtype_bytes != 2) return hipErrorInvalidValue;
+    const int vecs = (a.heads + 2 * a.kv_heads) * (a.head_dim / 16);
+    k_pf_qkv_post<bf16_t, true><<<a.M, std::min(512, (vecs + 63) / 64 * 64), 0, stream>>>(a);
+  } else if (dtype_bytes == 2) {
+    k_pf_qkv_post<bf16_t, false><<<a.M, 256, 0, stream>>>(a);
+  } else {
+    k_pf_qkv_post<float, false><<<a.M, 256, 0, stream>>>(a);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream) {
+template <int EPI, int MJ>
+static hipError_t gemm_launch(const GemmArgs& a, int splits, hipStream_t stream) {
+  constexpr int ST = gemm_stages(MJ), kLds = gemm_lds_bytes(MJ, ST);
+  constexpr int kTileN = EPI == kGemmSwiGlu ? kGn / 2 : kGn;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_bf16<EPI, MJ, ST>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  if (attr != hipSuccess) return attr;
+  const int nM = (a.M + gemm_tile_m(MJ) - 1) / gemm_tile_m(MJ), nN = (a.N + kTileN - 1) / kTileN;
+  k_gemm_bf16<EPI, MJ, ST><<<nM * nN * splits, kGthreads, kLds, stream>>>(a, nM, nN, splits);
+  return hipGetLastError();
+}
+template <int EPI>
+static hipError_t gemm_launch_mj(const GemmArgs& a, const GemmPlan& p, hipStream_t stream) {
+  switch (p.mj) {
+    case 1: return gemm_launch<EPI, 1>(a, p.splits, stream);
+    case 2: return gemm_launch<EPI, 2>(a, p.splits, stream);
+    case 3: return gemm_launch<EPI, 3>(a, p.splits, stream);
+    default: return gemm_launch<EPI, 4>(a, p.splits, stream);
+  }
+}
+
+// Tile height and K ranges of a bf16 GEMM: the pair with the least estimated
+// time, rounds x (K steps of a range x time per step + start and end) plus
+// the partial sums' write and read.  The times are fits to one MI355X at the
+// 7B projections, M = 10 .. 2,000 (steps of K = 64 with the tile's stages):
+// 0.66, 0.78, 1.25 and 1.3 us a step at 64, 128, 192 and 256 rows, about 4 us
+// a workgroup, partials at 2.2 TB/s through both kernels.  Ranges are taken
+// only while all of them fit one round (a second round of half-filled CUs
+// always lost: qkv at 120 tokens 13.3 us in 7 ranges, 20.2 in 8).
+// Measured, 256-row tiles without ranges against the plan's choice: 10
+// tokens, qkv 65 -> 9.0 us, o 65 -> 8.0, gate/up 83 -> 53, down 369 -> 26;
+// 570 tokens, qkv 66 -> 30, o 66 -> 23, gate/up 171 -> 166-174, down 355 ->
+// 81; from about 2,000 tokens on the 256-row tile without ranges is chosen.
+GemmPlan plan_gemm(int M, int N, int K, bool swiglu, size_t part_bytes) {
+  constexpr int kCus = 256;
+  constexpr double kStep[4] = {0.66, 0.78, 1.25, 1.3}, kFixed = 4.0, kPartBytesPerUs = 2.2e6;
+  const int steps = K / kGk, nN = (N + (swiglu ? kGn / 2 : kGn) - 1) / (swiglu ? kGn / 2 : kGn);
+  GemmPlan best{4, 1};
+  double best_us = 0;
+  for (int mj = 4; mj >= 1; --mj) {
+    const long long tiles = (long long)((M + gemm_tile_m(mj) - 1) / gemm_tile_m(mj)) * nN;
+    for (int s = 1; s <= steps; ++s) {
+      const size_t bytes = s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+      if (s > 1 && (swiglu || tiles * s > kCus || bytes > part_bytes)) break;
+      const double rounds = static_cast<double>((tiles * s + kCus - 1) / kCus);
+      const double us = rounds * ((steps + s - 1) / s * kStep[mj - 1] + kFixed) + bytes / kPartBytesPerUs;
+      if (best_us == 0 || us < best_us) {
+        best = GemmPlan{mj, s};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream, GemmPlan plan) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (dtype_bytes == 2) {
     const bool swiglu = epi == kGemmSwiGlu;
@@ -850,25 +1090,14 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t 
     if (a.K <= 0 || a.K % kGk != 0 || a.N % 8 != 0 || a.lda % 8 != 0 || a.ldw % 8 != 0 || a.ldo % 8 != 0 ||
         !aligned || (swiglu && a.W2 == nullptr))
       return hipErrorInvalidValue;
-    static const hipError_t attr = [] {
-      hipError_t e = hipSuccess;
-      for (const void* k : {reinterpret_cast<const void*>(k_gemm_bf16<kGemmStore>),
-                            reinterpret_cast<const void*>(k_gemm_bf16<kGemmResidual>),
-                            reinterpret_cast<const void*>(k_gemm_bf16<kGemmSwiGlu>)})
-        if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kGsmem);
-      return e;
-    }();
-    if (attr != hipSuccess) return attr;
-    const int tile_n = swiglu ? kGn / 2 : kGn;
-    const int nM = (a.M + kGm - 1) / kGm, nN = (a.N + tile_n - 1) / tile_n;
-    if (epi == kGemmStore)
-      k_gemm_bf16<kGemmStore><<<nM * nN, kGthreads, kGsmem, stream>>>(a, nM, nN);
-    else if (epi == kGemmResidual)
-      k_gemm_bf16<kGemmResidual><<<nM * nN, kGthreads, kGsmem, stream>>>(a, nM, nN);
-    else
-      k_gemm_bf16<kGemmSwiGlu><<<nM * nN, kGthreads, kGsmem, stream>>>(a, nM, nN);
+    const GemmPlan p = a.part != nullptr ? plan : plan_gemm(a.M, a.N, a.K, swiglu, 0);
+    if (p.mj < 1 || p.mj > 4 || p.splits < 1 || p.splits > a.K / kGk) return hipErrorInvalidValue;
+    if (a.part != nullptr) return gemm_launch_mj<kGemmPart>(a, p, stream);
+    if (epi == kGemmStore) return gemm_launch_mj<kGemmStore>(a, p, stream);
+    if (epi == kGemmResidual) return gemm_launch_mj<kGemmResidual>(a, p, stream);
+    return gemm_launch_mj<kGemmSwiGlu>(a, p, stream);
   } else {
-    if (a.K <= 0 || epi == kGemmSwiGlu) return hipErrorInvalidValue;
+    if (a.K <= 0 || epi == kGemmSwiGlu || a.part != nullptr) return hipErrorInvalidValue;
     const dim3 grid((a.N + 63) / 64, (a.M + 63) / 64);
     if (epi == kGemmStore)
       k_gemm_f32<kGemmStore><<<grid, 256, 0, stream>>>(a);

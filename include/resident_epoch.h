@@ -161,8 +161,9 @@ int32_t resident_epoch_prefill_batch(void *engine, int32_t n_rows,
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * Same arguments, checks and resulting state as resident_epoch_prefill_batch,
  * but the pass's activations and token tables live in a fixed 64 MiB device
- * array of the library (one per GPU, held until the process ends) instead of
- * the engine's grown-on-demand buffer.  Calls on
+ * array of the library (one per GPU, held until the process ends; 64 MiB more
+ * behind it hold the partial sums of split products) instead of the engine's
+ * grown-on-demand buffer.  Calls on
  * one GPU share the array and are serialized; a call leaves its contents
  * behind.  The array's device address is resolved on the first call on a
  * device (no allocation).  Return 0, -1 bad arguments, -2 HIP failure
