@@ -271,7 +271,7 @@ int balance(int groups, int resident) {
   return (groups + iters - 1) / iters;
 }
 
-bool make_plan(Engine& e, const Json& cfg) {
+bool make_plan(Engine& e, const Json& cfg, bool packed) {
   const Dims& d = e.dims;
   LaunchPlan& p = e.plan;
   p.mb = d.batch <= 4 ? 4 : 8;
@@ -294,14 +294,19 @@ bool make_plan(Engine& e, const Json& cfg) {
   if (const Json* t = cfg.get("tuning"))
     if (t->number_or("qkv_ksplit", 1) == 0) p.qkv_ksplit = 0;
   const Json* tune = cfg.get("tuning");
-  // 64 bf16 rows of Qwen2.5-7B's shape: projections on the matrix cores,
+  // 5 to 64 bf16 rows of Qwen2.5-7B's shape: projections on the matrix cores,
   // gate/up and the LM head one workgroup per CU, qkv, o and down split over
   // (strip group, K range) (re_mfma.hip); "tuning": {"mfma": 0} keeps the
-  // row-tiled kernels
+  // row-tiled kernels, and so does an engine without the memory for the
+  // packed weights.  The row-tiled kernels read every weight once per 8 rows:
+  // a step of one layer and the LM head at 16 rows took 600 us there and
+  // takes 312 here, two layers and the head at 41 rows 2,229 and 481.  At up
+  // to four rows the four-row kernels stream the weights once and need no
+  // partial sums.
   p.mfma = 0;
   p.gu_cu = 0;
-  if (mfma_step_supported(d) && mfma_lm_cu_fits(d, e.cus) && mfma_gu_cu_fits(d, e.cus) && mfma_qkv_split_fits(d) &&
-      (tune == nullptr || tune->number_or("mfma", 1) != 0) && prepare_mfma() == hipSuccess) {
+  if (packed && mfma_step_supported(d) && mfma_lm_cu_fits(d, e.cus) && mfma_gu_cu_fits(d, e.cus) && mfma_qkv_split_fits(d) &&
+      (tune == nullptr || tune->number_or("mfma", 1) != 0) && prepare_mfma(d) == hipSuccess) {
     p.mfma = 1;
     p.gu_cu = e.cus;
     p.lm_wg = e.cus;  // k_mf_lm_cu's workgroups
@@ -500,11 +505,12 @@ bool alloc_state(Engine& e) {
     void** p;
     size_t bytes;
   };
+  const size_t XB = p.mfma ? mfma_padded_rows(d) : B;  // rows of the projections' (packed) inputs
   std::vector<Part> sp = {
       {&e.scratch.hidden, (size_t)B * d.hidden * T},
       {&e.scratch.q, (size_t)B * d.q_dim() * T},
-      {&e.scratch.attn, (size_t)B * d.q_dim() * T},
-      {&e.scratch.mlp, (size_t)B * d.intermediate * T},
+      {&e.scratch.attn, XB * d.q_dim() * T},
+      {&e.scratch.mlp, XB * d.intermediate * T},
       {reinterpret_cast<void**>(&e.scratch.partial),
        (size_t)std::max(p.down_segments, p.o_segments) * B * d.hidden * sizeof(float)},
       {reinterpret_cast<void**>(&e.scratch.am_val), (size_t)p.lm_wg * B * sizeof(float)},
@@ -512,7 +518,7 @@ bool alloc_state(Engine& e) {
       {reinterpret_cast<void**>(&e.scratch.am_bad), (size_t)p.lm_wg * B * sizeof(int32_t)},
       {reinterpret_cast<void**>(&e.scratch.inv_freq), (size_t)d.head_dim / 2 * sizeof(float)},
       {reinterpret_cast<void**>(&e.scratch.rope), (size_t)B * d.head_dim * sizeof(float)},
-      {&e.scratch.xn, p.mfma ? (size_t)B * d.hidden * T : 0},
+      {&e.scratch.xn, p.mfma ? XB * d.hidden * T : 0},
       {reinterpret_cast<void**>(&e.scratch.mf_part), p.mfma ? mfma_split_partial_bytes(d) : 0},
       {reinterpret_cast<void**>(&e.scratch.sp_scores), (size_t)p.attn_split * 256 * B * d.heads * sizeof(float)},
       {reinterpret_cast<void**>(&e.scratch.sp_stats), (size_t)p.attn_split * 2 * B * d.heads * sizeof(float)},
@@ -575,6 +581,24 @@ bool alloc_state(Engine& e) {
   std::memset(e.h_feed, 0, e.import_feed_bytes);
   std::memset(e.h_fetch, 0, e.fetch_bytes);
   return true;
+}
+
+// The packed copy of the projections (matrix-core plan).  Below 64 rows it is
+// taken only while the buffers that grow later (the decoder-step caches, a
+// prefill of every row's window) still fit beside it.
+bool alloc_packed(Engine& e) {
+  if (!e.plan.mfma) return true;
+  const Dims& d = e.dims;
+  e.packed_off.resize(d.layers);
+  const size_t bytes = mfma_packed_layout(d, e.packed_off.data(), &e.packed_lm_off);
+  if (d.batch < 64) {
+    const size_t token = (2 * (size_t)d.hidden + d.qkv_rows() + d.q_dim() + d.intermediate) * d.dtype_bytes +
+                         (size_t)d.head_dim * sizeof(float) + 64;
+    const size_t later = 2 * e.cache_bytes + (size_t)d.batch * d.capacity * token + kPrefillPartBytes + (1ull << 30);
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < bytes + later) return false;
+  }
+  return hipMalloc(&e.packed, bytes) == hipSuccess;
 }
 
 bool load_bundle(Engine& e, const std::string& dir) {
@@ -741,22 +765,35 @@ void drop_graphs(Engine& e) {
   e.graph_defs.clear();
 }
 
+// What alloc_state and alloc_packed allocated.
+void free_state(Engine& e) {
+  auto drop = [](auto& p) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  };
+  auto drop_host = [](auto& p) {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+  };
+  drop(e.packed);
+  drop(e.key_cache);
+  drop(e.value_cache);
+  drop(e.state_mem);
+  drop(e.scratch_mem);
+  drop(e.step_mem);
+  drop_host(e.h_feed);
+  drop_host(e.h_fetch);
+}
+
 void free_engine(Engine* e) {
   if (!e) return;
   drop_graphs(*e);
   if (e->ev_start) (void)hipEventDestroy(e->ev_start);
   if (e->ev_stop) (void)hipEventDestroy(e->ev_stop);
   if (e->weights) (void)hipFree(e->weights);
-  if (e->packed) (void)hipFree(e->packed);
-  if (e->key_cache) (void)hipFree(e->key_cache);
-  if (e->value_cache) (void)hipFree(e->value_cache);
-  if (e->state_mem) (void)hipFree(e->state_mem);
-  if (e->scratch_mem) (void)hipFree(e->scratch_mem);
-  if (e->step_mem) (void)hipFree(e->step_mem);
+  free_state(*e);
   if (e->dec_key) (void)hipFree(e->dec_key);
   if (e->dec_value) (void)hipFree(e->dec_value);
-  if (e->h_feed) (void)hipHostFree(e->h_feed);
-  if (e->h_fetch) (void)hipHostFree(e->h_fetch);
   for (auto& kv : e->ipc_maps) (void)hipIpcCloseMemHandle(kv.second.ptr);
   if (e->pf_mem) (void)hipFree(e->pf_mem);
   if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1008,26 +1045,28 @@ extern "C" void* resident_epoch_create(const char* air_path, const char* graph_c
     *status = kCreateRuntime;
     return nullptr;
   }
-  if (!make_plan(*e, cfg)) {
+  if (!make_plan(*e, cfg, true)) {
     *status = kCreateGraph;
     return nullptr;
   }
   layout_weights(*e);
-  if (hipMalloc(&e->weights, e->weight_bytes) != hipSuccess || !alloc_state(*e)) {
+  if (hipMalloc(&e->weights, e->weight_bytes) != hipSuccess) {
     *status = kCreateDevice;
     return nullptr;
+  }
+  if (!alloc_state(*e) || !alloc_packed(*e)) {
+    // without the room for the packed weights below 64 rows: the row-tiled plan
+    const bool retry = e->plan.mfma && e->dims.batch < 64;
+    free_state(*e);
+    (void)hipGetLastError();
+    if (!retry || !make_plan(*e, cfg, false) || !alloc_state(*e)) {
+      *status = kCreateDevice;
+      return nullptr;
+    }
   }
   if (hipMemset(e->weights, 0, e->weight_bytes) != hipSuccess) {
     *status = kCreateDevice;
     return nullptr;
-  }
-  if (e->plan.mfma) {
-    e->packed_off.resize(e->dims.layers);
-    const size_t packed_bytes = mfma_packed_layout(e->dims, e->packed_off.data(), &e->packed_lm_off);
-    if (hipMalloc(&e->packed, packed_bytes) != hipSuccess) {
-      *status = kCreateDevice;
-      return nullptr;
-    }
   }
   const Json* w = cfg.get("weights");
   const std::string source = w ? w->string_or("source", "bundle") : "bundle";

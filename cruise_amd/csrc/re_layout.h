@@ -239,7 +239,10 @@ bool mfma_split_fits(const Dims& d);
 bool mfma_gu_cu_fits(const Dims& d, int cus);
 size_t mfma_split_partial_bytes(const Dims& d);
 bool mfma_qkv_split_fits(const Dims& d);
-hipError_t prepare_mfma();
+hipError_t prepare_mfma(const Dims& d);
+// Rows of the packed activations (whole 16-row tiles; rows past the batch are
+// read but reach no output).
+int mfma_padded_rows(const Dims& d);
 // Layout of the packed copy; returns its bytes.
 size_t mfma_packed_layout(const Dims& d, PackedOffsets* layers, size_t* lm_off);
 // Pack one [rows, K] matrix (qkv_head_dim > 0: the stacked qkv matrix, whose

@@ -1,11 +1,13 @@
 // Decode projections of the resident epoch on the matrix cores (gfx950), for
-// 64 batch rows (the scaled-batch configuration): Y[B, N] = X[B, K] W[N, K]^T
-// with v_mfma_f32_16x16x32_bf16, the weights streamed from HBM once per step.
+// 5 to 64 batch rows: Y[B, N] = X[B, K] W[N, K]^T with
+// v_mfma_f32_16x16x32_bf16, the weights streamed from HBM once per step.  The
+// kernels are compiled for TT = 1 .. 4 16-row batch tiles; the rows that fill
+// up the last tile hold whatever the buffers hold and reach no output.
 //
 // Work layout.  Weights stream as 16-row column strips: lane l holds row
 // l % 16 of the strip and elements 8 (l / 16) ..+8 of each 32-wide k step (a
 // 64-byte run per row per load instruction; the packed copy makes a wave's
-// step one 1 KB run), against the matching activation fragments of the four
+// step one 1 KB run), against the matching activation fragments of the TT
 // 16-row batch tiles, staged once per CU in LDS.  Weights are requested kRing
 // (or more) steps ahead with every wait count known at compile time.
 //   LM head, gate/up  one workgroup per CU, each wave a strip (two for
@@ -38,8 +40,8 @@ namespace {
 typedef __bf16 mf_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mf_f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMfRows = 64;   // batch rows of the configuration
-constexpr int kMfTiles = kMfRows / 16;
+constexpr int kMfRows = 64;   // batch rows at most
+constexpr int kMfMinRows = 5;  // fewer take the four-row kernels of re_step.hip
 constexpr int kMfK = 32;      // k per MFMA step
 constexpr int kRing = 8;      // weight steps in flight per wave
 // Qwen2.5-7B's shape, the one these instantiations are compiled for
@@ -88,23 +90,28 @@ __device__ __forceinline__ int qkv_strip_row(int head_dim, int g, int c) {
 // Packed activations: xpack_index (re_device.h).
 
 // LM head with one workgroup per CU.  Workgroups of a few waves would each
-// fetch the whole 64 x K activation block (with 4-wave workgroups, 0.7 GB per
-// step on top of the 1.09 GB of weights); here the 8 waves of a CU's one
-// workgroup share one copy, staged through LDS in blocks of 16 k steps
-// (64 KB, two buffers, filled by global -> LDS loads).  Workgroup g owns
+// fetch the whole B x K activation block (at 64 rows with 4-wave workgroups,
+// 0.7 GB per step on top of the 1.09 GB of weights); here the 8 waves of a
+// CU's one workgroup share one copy, staged through LDS in blocks of 16 (one
+// and two tiles: 56 and 28) k steps (up to 64 KB, two buffers, filled by
+// global -> LDS loads).  Workgroup g owns
 // strips [g T / G, (g + 1) T / G) of the T = V / 16 column strips; wave w
 // owns strips w, w + 8, ... of that range (NS = 4 or 5 of them) over the whole
 // K, with kLcRing k steps of weights in flight.  Per step a wave reads the
 // four batch tiles' fragments from LDS and runs NS x 4 products, every logit
 // one chain of MFMA steps in k order; the argmax partial of (workgroup, row) is the first
 // index of the maximum over the workgroup's columns (CTRL:99-119), combined
-// over the waves in wave order, stored row-major ([row][G]).
+// over the waves in wave order, stored row-major ([row][G]).  Bound by HBM:
+// 166 us at 16 rows, 171 at 41 and 179 at 64 (6.6, 6.4 and 6.1 TB/s); the
+// row-tiled kernel took 357, 1,059 and 1,420.
 constexpr int kLcWaves = 8;
-constexpr int kLcBlock = 16;   // k steps per LDS activation block
 constexpr int kLcRing = 4;     // weight steps in flight per wave
 constexpr int kLcMaxNs = 5;    // strips per wave at most
-constexpr int kLcBlockBytes = kMfTiles * kLcBlock * 1024;
-constexpr size_t kLcLds = 2 * (size_t)kLcBlockBytes + (size_t)kLcWaves * kMfRows * 12;
+// k steps per LDS activation block at TT 16-row batch tiles: up to 64 KB
+constexpr int lc_block(int tt) { return tt == 1 ? 56 : tt == 2 ? 28 : 16; }
+constexpr int lc_block_bytes(int tt) { return tt * lc_block(tt) * 1024; }
+constexpr int kLcMaxBlock = 56;
+constexpr size_t lc_lds(int tt) { return 2 * (size_t)lc_block_bytes(tt) + (size_t)kLcWaves * kMfRows * 12; }
 
 typedef const __attribute__((address_space(1))) void* lc_gptr;
 typedef __attribute__((address_space(3))) void* lc_lptr;
@@ -118,30 +125,35 @@ constexpr int lc_wait(int vm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4);
 // each, packed) with RING steps in flight, accumulating acc[j][t] over the
 // whole K in step order.  NS = 0: a wave with no strip only loads and joins
 // the barriers (every wave runs the same 1 + K / (32 kLcBlock) barriers).
-template <int NS, int RING>
+template <int TT, int NS, int RING>
 __device__ __forceinline__ void cu_stream(const MfArgs& a, unsigned char* lds, const bf16_t* const* wp, int lane,
-                                          int wave, mf_f32x4 (*acc)[kMfTiles]) {
+                                          int wave, mf_f32x4 (*acc)[TT]) {
   constexpr int NA = NS > 0 ? NS : 1;
-  static_assert(RING * NS + 8 <= 63, "vmcnt holds at most 63");
+  constexpr int kLcBlock = lc_block(TT), kLcBlockBytes = lc_block_bytes(TT);
+  constexpr int kCopies = TT * kLcBlock / kLcWaves;  // activation loads per wave and block
+  static_assert(TT * kLcBlock % kLcWaves == 0, "every wave copies the same number of fragments");
+  static_assert(RING * NS + kCopies <= 63, "vmcnt holds at most 63");
   static_assert(kLcBlock % RING == 0, "ring slots are compile-time within a block");
   const int ksteps = a.K / kMfK, nblocks = ksteps / kLcBlock;
-  // activation block b, tile t, steps 8 (w & 1) ..+8 go to LDS by wave w's 8
-  // loads (load i: step s0 + i)
+  // fragments kCopies w ..+kCopies of activation block b (tile-major) go to
+  // LDS by wave w's loads
+  constexpr bool kOneTile = kLcBlock % kCopies == 0;  // a wave's fragments lie in one tile
+  const int f0 = wave * kCopies, t0 = f0 / kLcBlock, s0 = f0 - t0 * kLcBlock;
   auto issue_x1 = [&](int b, int i) {
-    const int t = wave >> 1, s0 = (wave & 1) * 8;
-    const bf16_t* src = a.x + ((size_t)t * ksteps + b * kLcBlock + s0 + i) * 512 + lane * 8;
-    unsigned char* dst = lds + (b & 1) * kLcBlockBytes + (t * kLcBlock + s0 + i) * 1024;
+    const int t = kOneTile ? t0 : (f0 + i) / kLcBlock, s = kOneTile ? s0 + i : f0 + i - t * kLcBlock;
+    const bf16_t* src = a.x + ((size_t)t * ksteps + b * kLcBlock + s) * 512 + lane * 8;
+    unsigned char* dst = lds + (b & 1) * kLcBlockBytes + (f0 + i) * 1024;
     __builtin_amdgcn_global_load_lds((lc_gptr)src, (lc_lptr)dst, 16, 0, 0);
   };
   auto issue_x = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) issue_x1(b, i);
+    for (int i = 0; i < kCopies; ++i) issue_x1(b, i);
   };
   if constexpr (NS > 0) {
 #pragma unroll
     for (int j = 0; j < NS; ++j)
 #pragma unroll
-      for (int t = 0; t < kMfTiles; ++t) acc[j][t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < TT; ++t) acc[j][t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   re_u32x4 wr[RING][NA];
   issue_x(0);
@@ -152,23 +164,19 @@ __device__ __forceinline__ void cu_stream(const MfArgs& a, unsigned char* lds, c
       for (int j = 0; j < NS; ++j) wr[s][j] = __builtin_nontemporal_load(reinterpret_cast<const re_u32x4*>(wp[j] + s * 512));
   }
   // Block b + 1 goes to LDS during block b (its buffer was freed by the
-  // barrier that ended block b - 1).  SPREAD (a ring no deeper than the
-  // block's last 8 steps): one load per step over the block's first 8
-  // steps, so no wave stalls on a burst of eight requests, and at least RING
-  // steps of refills follow the last one, so the block-end wait (all but the
-  // last RING * NS loads) covers it; a wave without strips issues them at
-  // the block's start.  Otherwise (a deeper ring, whose block-end wait
-  // leaves loads of the whole block in flight): block b + 2 in one burst
-  // after the barrier that ends block b.
-  constexpr bool SPREAD = RING <= kLcBlock - 8;
-  if constexpr (!SPREAD) issue_x(1);
-  // block 0 in LDS (the ring, and block 1 without SPREAD, may still be in flight)
+  // barrier that ended block b - 1): one load per step over the block's first
+  // kCopies steps, so no wave stalls on a burst of requests, and at least
+  // RING steps of refills follow the last one, so the block-end wait (all but
+  // the last RING * NS loads) covers it; a wave without strips issues them at
+  // the block's start.
+  static_assert(RING + kCopies <= kLcBlock, "RING steps of refills follow a block's copies");
+  // block 0 in LDS (the ring may still be in flight)
   asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(lc_wait(RING * NS + (SPREAD ? 0 : 8)));
+  __builtin_amdgcn_s_waitcnt(lc_wait(RING * NS));
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   for (int b = 0; b < nblocks; ++b) {
-    if constexpr (SPREAD && NS == 0) {
+    if constexpr (NS == 0) {
       if (b + 1 < nblocks) issue_x(b + 1);
     }
     if constexpr (NS > 0) {
@@ -176,20 +184,20 @@ __device__ __forceinline__ void cu_stream(const MfArgs& a, unsigned char* lds, c
 #pragma unroll
       for (int s = 0; s < kLcBlock; ++s) {
         const int S = b * kLcBlock + s, rw = S % RING;
-        mf_bf16x8 xf[kMfTiles];
+        mf_bf16x8 xf[TT];
 #pragma unroll
-        for (int t = 0; t < kMfTiles; ++t) xf[t] = *reinterpret_cast<const mf_bf16x8*>(xb + (t * kLcBlock + s) * 1024);
+        for (int t = 0; t < TT; ++t) xf[t] = *reinterpret_cast<const mf_bf16x8*>(xb + (t * kLcBlock + s) * 1024);
 #pragma unroll
         for (int j = 0; j < NS; ++j)
 #pragma unroll
-          for (int t = 0; t < kMfTiles; ++t)
+          for (int t = 0; t < TT; ++t)
             acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[t], __builtin_bit_cast(mf_bf16x8, wr[rw][j]), acc[j][t], 0, 0, 0);
         // the refill past the last step re-reads the last one (unconditional,
         // so every wait counts exactly these loads)
         const int nxt = min(S + RING, ksteps - 1);
 #pragma unroll
         for (int j = 0; j < NS; ++j) wr[rw][j] = __builtin_nontemporal_load(reinterpret_cast<const re_u32x4*>(wp[j] + nxt * 512));
-        if (SPREAD && s < 8 && b + 1 < nblocks) issue_x1(b + 1, s);
+        if (s < kCopies && b + 1 < nblocks) issue_x1(b + 1, s);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -199,25 +207,24 @@ __device__ __forceinline__ void cu_stream(const MfArgs& a, unsigned char* lds, c
     __builtin_amdgcn_s_waitcnt(lc_wait(RING * NS));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (!SPREAD && b + 2 < nblocks) issue_x(b + 2);
   }
   __builtin_amdgcn_s_waitcnt(lc_wait(0));
 }
 
-template <int NS>
+template <int TT, int NS>
 __device__ __forceinline__ void lm_cu_body(const MfArgs& a, unsigned char* lds, int s_begin, int lane, int wave,
                                            float* cval, int* cidx, int* cbad) {
   const int ksteps = a.K / kMfK;
   const bf16_t* wp[NS];
 #pragma unroll
   for (int j = 0; j < NS; ++j) wp[j] = a.p0 + (size_t)(s_begin + wave + kLcWaves * j) * ksteps * 512 + lane * 8;
-  mf_f32x4 acc[NS][kMfTiles];
-  cu_stream<NS, kLcRing>(a, lds, wp, lane, wave, acc);
+  mf_f32x4 acc[NS][TT];
+  cu_stream<TT, NS, kLcRing>(a, lds, wp, lane, wave, acc);
   // Logits T(y) as fp32 (batched_decoder_step.py:405-408) and this wave's
   // first maximum per row over its strips.
   const int c = lane & 15, mrow = 4 * (lane >> 4);
 #pragma unroll
-  for (int t = 0; t < kMfTiles; ++t)
+  for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int m = t * 16 + mrow + v;
@@ -252,6 +259,7 @@ __device__ __forceinline__ void lm_cu_body(const MfArgs& a, unsigned char* lds, 
     }
 }
 
+template <int TT>
 __global__ void __launch_bounds__(kLcWaves * 64, 1) k_mf_lm_cu(MfArgs a) {
   extern __shared__ __align__(16) unsigned char lc_smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
@@ -260,16 +268,16 @@ __global__ void __launch_bounds__(kLcWaves * 64, 1) k_mf_lm_cu(MfArgs a) {
   const int G = gridDim.x, g = blockIdx.x, T = a.vocab / 16;
   const int s_begin = (int)((long long)g * T / G), s_end = (int)((long long)(g + 1) * T / G);
   const int ns = (s_end - s_begin - wave + kLcWaves - 1) / kLcWaves;  // strips of this wave
-  float* cval = reinterpret_cast<float*>(lc_smem + 2 * (size_t)kLcBlockBytes);
+  float* cval = reinterpret_cast<float*>(lc_smem + 2 * (size_t)lc_block_bytes(TT));
   int* cidx = reinterpret_cast<int*>(cval + kLcWaves * kMfRows);
   int* cbad = cidx + kLcWaves * kMfRows;
   // every wave runs the same barriers whatever its strip count
   switch (ns) {
-    case 5: lm_cu_body<5>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
-    case 4: lm_cu_body<4>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
-    case 3: lm_cu_body<3>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
-    case 2: lm_cu_body<2>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
-    default: lm_cu_body<1>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;  // ns >= 1 (launch check)
+    case 5: lm_cu_body<TT, 5>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
+    case 4: lm_cu_body<TT, 4>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
+    case 3: lm_cu_body<TT, 3>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
+    case 2: lm_cu_body<TT, 2>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;
+    default: lm_cu_body<TT, 1>(a, lc_smem, s_begin, lane, wave, cval, cidx, cbad); break;  // ns >= 1 (launch check)
   }
   __syncthreads();
   if (tid < a.B) {
@@ -291,13 +299,15 @@ __global__ void __launch_bounds__(kLcWaves * 64, 1) k_mf_lm_cu(MfArgs a) {
   }
 }
 
-// gate/up with one workgroup per CU (64 rows): the I / 16 column strips are
+// gate/up with one workgroup per CU: the I / 16 column strips are
 // split over the CUs (4-5 each for Qwen2.5-7B), wave w < that count streams
 // strip s_begin + w of the gate and of the up matrix over the whole K,
 // sharing the LDS-staged activations with the other waves, then the SiLU *
-// up epilogue.
-constexpr int kGcRing = 8;  // weight steps in flight per wave (few waves stream)
+// up epilogue.  47 us at 16 rows, 50 at 41, 52 at 64 (row-tiled: 93, 266, -).
+// weight steps in flight per wave (few waves stream)
+constexpr int gc_ring(int tt) { return tt <= 2 ? 14 : 8; }
 
+template <int TT>
 __global__ void __launch_bounds__(kLcWaves * 64, 1) k_mf_gu_cu(MfArgs a) {
   extern __shared__ __align__(16) unsigned char lc_smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
@@ -307,16 +317,16 @@ __global__ void __launch_bounds__(kLcWaves * 64, 1) k_mf_gu_cu(MfArgs a) {
   const int s_begin = (int)((long long)g * T / G), s_end = (int)((long long)(g + 1) * T / G);
   const int u = s_begin + wave;
   if (u >= s_end) {
-    cu_stream<0, kGcRing>(a, lc_smem, nullptr, lane, wave, nullptr);
+    cu_stream<TT, 0, gc_ring(TT)>(a, lc_smem, nullptr, lane, wave, nullptr);
     return;
   }
   const int ksteps = a.K / kMfK;
   const bf16_t* wp[2] = {a.p0 + (size_t)u * ksteps * 512 + lane * 8, a.p1 + (size_t)u * ksteps * 512 + lane * 8};
-  mf_f32x4 acc[2][kMfTiles];
-  cu_stream<2, kGcRing>(a, lc_smem, wp, lane, wave, acc);
+  mf_f32x4 acc[2][TT];
+  cu_stream<TT, 2, gc_ring(TT)>(a, lc_smem, wp, lane, wave, acc);
   const int c = lane & 15, mrow = 4 * (lane >> 4), n = u * 16 + c;
 #pragma unroll
-  for (int t = 0; t < kMfTiles; ++t)
+  for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int m = t * 16 + mrow + v;
@@ -344,9 +354,9 @@ template <int STEPS, int BLK>
 constexpr int part_block_steps(int b) {
   return STEPS - b * BLK < BLK ? STEPS - b * BLK : BLK;
 }
-template <int STEPS, int BLK, int WAVES>
+template <int TT, int STEPS, int BLK, int WAVES>
 constexpr int part_block_copies(int b) {  // per wave
-  return (kMfTiles * part_block_steps<STEPS, BLK>(b) + WAVES - 1) / WAVES;
+  return (TT * part_block_steps<STEPS, BLK>(b) + WAVES - 1) / WAVES;
 }
 template <int STEPS, int BLK>
 constexpr int part_block_refills(int b) {  // weight loads issued during block b
@@ -354,17 +364,17 @@ constexpr int part_block_refills(int b) {  // weight loads issued during block b
   for (int s = b * BLK; s < b * BLK + part_block_steps<STEPS, BLK>(b); ++s) n += s + kRing < STEPS ? 1 : 0;
   return n;
 }
-template <int STEPS, int BLK>
+template <int TT, int STEPS, int BLK>
 constexpr size_t part_cu_lds() {
-  return (size_t)(STEPS > BLK ? 2 : 1) * kMfTiles * BLK * 1024;
+  return (size_t)(STEPS > BLK ? 2 : 1) * TT * BLK * 1024;
 }
 
-template <int STEPS, int WAVES, int BLK, bool QKV>
+template <int TT, int STEPS, int WAVES, int BLK, bool QKV>
 __global__ void __launch_bounds__(WAVES * 64) k_mf_part_cu(MfArgs a) {
-  extern __shared__ __align__(16) unsigned char pc_smem[];  // [2][kMfTiles][BLK] fragments of 1 KB
+  extern __shared__ __align__(16) unsigned char pc_smem[];  // [2][TT][BLK] fragments of 1 KB
   constexpr int NB = (STEPS + BLK - 1) / BLK;
   constexpr int R = kRing < STEPS ? kRing : STEPS;
-  constexpr int kBuf = kMfTiles * BLK * 1024;
+  constexpr int kBuf = TT * BLK * 1024;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
   const int c = lane & 15;
   const int g = blockIdx.x * WAVES + wave;  // this wave's strip
@@ -377,10 +387,10 @@ __global__ void __launch_bounds__(WAVES * 64) k_mf_part_cu(MfArgs a) {
   auto stage = [&](auto bc) {
     constexpr int b = decltype(bc)::value;
     constexpr int ns = part_block_steps<STEPS, BLK>(b);
-    constexpr int nf = kMfTiles * ns;
+    constexpr int nf = TT * ns;
     unsigned char* dst = pc_smem + (b & 1) * kBuf;
 #pragma unroll
-    for (int i = 0; i < part_block_copies<STEPS, BLK, WAVES>(b); ++i) {
+    for (int i = 0; i < part_block_copies<TT, STEPS, BLK, WAVES>(b); ++i) {
       const int f = min(wave + i * WAVES, nf - 1);
       const int t = f / ns, sl = f - t * ns;
       __builtin_amdgcn_global_load_lds((lc_gptr)(a.x + ((size_t)t * ksteps + kstep0 + b * BLK + sl) * 512 + lane * 8),
@@ -395,17 +405,17 @@ __global__ void __launch_bounds__(WAVES * 64) k_mf_part_cu(MfArgs a) {
   int pending = R;  // loads issued after the block now awaited (compile-time after unrolling)
   if constexpr (NB > 1) {
     stage(std::integral_constant<int, 1>{});
-    pending += part_block_copies<STEPS, BLK, WAVES>(1);
+    pending += part_block_copies<TT, STEPS, BLK, WAVES>(1);
   }
   // block 0 is in LDS: this wave's copies first, then everyone's
   asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(lc_wait(R + (NB > 1 ? part_block_copies<STEPS, BLK, WAVES>(1) : 0)));
+  __builtin_amdgcn_s_waitcnt(lc_wait(R + (NB > 1 ? part_block_copies<TT, STEPS, BLK, WAVES>(1) : 0)));
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   (void)pending;
-  mf_f32x4 acc[kMfTiles];
+  mf_f32x4 acc[TT];
 #pragma unroll
-  for (int t = 0; t < kMfTiles; ++t) acc[t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < TT; ++t) acc[t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
   auto block = [&](auto bc) {
     constexpr int b = decltype(bc)::value;
     constexpr int ns = part_block_steps<STEPS, BLK>(b);
@@ -413,11 +423,11 @@ __global__ void __launch_bounds__(WAVES * 64) k_mf_part_cu(MfArgs a) {
 #pragma unroll
     for (int sl = 0; sl < ns; ++sl) {
       const int s = b * BLK + sl;
-      mf_bf16x8 xf[kMfTiles];
+      mf_bf16x8 xf[TT];
 #pragma unroll
-      for (int t = 0; t < kMfTiles; ++t) xf[t] = *reinterpret_cast<const mf_bf16x8*>(xb + (t * BLK + sl) * 1024);
+      for (int t = 0; t < TT; ++t) xf[t] = *reinterpret_cast<const mf_bf16x8*>(xb + (t * BLK + sl) * 1024);
 #pragma unroll
-      for (int t = 0; t < kMfTiles; ++t)
+      for (int t = 0; t < TT; ++t)
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[t], __builtin_bit_cast(mf_bf16x8, wr[s % R]), acc[t], 0, 0, 0);
       if (s + R < STEPS) wr[s % R] = __builtin_nontemporal_load(reinterpret_cast<const re_u32x4*>(wp + (s + R) * 512));
       __builtin_amdgcn_sched_barrier(0);
@@ -443,7 +453,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_mf_part_cu(MfArgs a) {
   const int n = QKV ? qkv_strip_row(a.head_dim, g, c) : g * 16 + c;
   float* part = a.part + (size_t)blockIdx.y * a.B * a.hidden_dim;
 #pragma unroll
-  for (int t = 0; t < kMfTiles; ++t)
+  for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int m = t * 16 + mrow + v;
@@ -603,8 +613,21 @@ constexpr int kDownBlk = 16;
 
 }  // namespace
 
+// Calls f with the number of 16-row tiles of B batch rows (1 to 4).
+template <typename F>
+static void mf_tiles(int B, F f) {
+  switch ((B + 15) / 16) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    default: f(std::integral_constant<int, 4>{}); break;
+  }
+}
+
+int mfma_padded_rows(const Dims& d) { return (d.batch + 15) / 16 * 16; }
+
 bool mfma_step_supported(const Dims& d) {
-  return d.dtype_bytes == 2 && d.batch == kMfRows && d.hidden == kMfHidden && d.q_dim() == kMfHidden &&
+  return d.dtype_bytes == 2 && d.batch >= kMfMinRows && d.batch <= kMfRows && d.hidden == kMfHidden && d.q_dim() == kMfHidden &&
          d.intermediate == kMfInter && d.head_dim % 16 == 0 && d.qkv_rows() % 16 == 0 &&
          d.vocab % 32 == 0 && d.hidden % 16 == 0;
 }
@@ -615,7 +638,7 @@ int mfma_lm_partials(const Dims& d) { return d.vocab / 32; }
 bool mfma_gu_cu_fits(const Dims& d, int cus) {
   const int strips = d.intermediate / 16;
   return mfma_step_supported(d) && cus > 0 && strips >= cus && strips <= kLcWaves * cus &&
-         d.hidden % (kMfK * kLcBlock) == 0 && d.hidden / (kMfK * kLcBlock) >= 2;
+         d.hidden % (kMfK * kLcMaxBlock) == 0 && d.hidden / (kMfK * kLcMaxBlock) >= 2;
 }
 
 bool mfma_split_fits(const Dims& d) { return mfma_step_supported(d) && (d.hidden / 16) % kPartWaves == 0; }
@@ -630,7 +653,7 @@ size_t mfma_split_partial_bytes(const Dims& d) {
 bool mfma_lm_cu_fits(const Dims& d, int cus) {
   const int strips = d.vocab / 16;
   return mfma_step_supported(d) && cus > 0 && strips >= kLcWaves * cus && strips <= kLcWaves * kLcMaxNs * cus &&
-         d.hidden % (kMfK * kLcBlock) == 0 && d.hidden / (kMfK * kLcBlock) >= 2 && cus <= mfma_lm_partials(d);
+         d.hidden % (kMfK * kLcMaxBlock) == 0 && d.hidden / (kMfK * kLcMaxBlock) >= 2 && cus <= mfma_lm_partials(d);
 }
 
 size_t mfma_packed_layout(const Dims& d, PackedOffsets* layers, size_t* lm_off) {
@@ -659,25 +682,37 @@ hipError_t mfma_pack_matrix(const void* src, void* dst, int rows, int K, int qkv
   return hipGetLastError();
 }
 
-template <int STEPS, int WAVES, int BLK, bool QKV>
+template <int TT, int STEPS, int WAVES, int BLK, bool QKV>
 static hipError_t part_cu_prepare() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_part_cu<STEPS, WAVES, BLK, QKV>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part_cu_lds<STEPS, BLK>()));
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_part_cu<TT, STEPS, WAVES, BLK, QKV>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             static_cast<int>(part_cu_lds<TT, STEPS, BLK>()));
 }
 template <int STEPS, int WAVES, int BLK, bool QKV>
 static void part_cu_launch(const MfArgs& a, int groups, hipStream_t stream) {
-  k_mf_part_cu<STEPS, WAVES, BLK, QKV><<<dim3(groups, kPartRanges), WAVES * 64, part_cu_lds<STEPS, BLK>(), stream>>>(a);
+  mf_tiles(a.B, [&](auto tt) {
+    constexpr int TT = decltype(tt)::value;
+    k_mf_part_cu<TT, STEPS, WAVES, BLK, QKV>
+        <<<dim3(groups, kPartRanges), WAVES * 64, part_cu_lds<TT, STEPS, BLK>(), stream>>>(a);
+  });
 }
 
-hipError_t prepare_mfma() {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_lm_cu), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     static_cast<int>(kLcLds));
+template <int TT>
+static hipError_t prepare_tiles() {
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_lm_cu<TT>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lc_lds(TT)));
   if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_gu_cu), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(kLcLds));
-  if (e == hipSuccess) e = part_cu_prepare<kHidSteps(kPartRanges), kPartWaves, kHidSteps(kPartRanges), false>();
-  if (e == hipSuccess) e = part_cu_prepare<kInterSteps, kPartWaves, kDownBlk, false>();
-  if (e == hipSuccess) e = part_cu_prepare<kHidSteps(kPartRanges), kQkvPartWaves, kHidSteps(kPartRanges), true>();
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mf_gu_cu<TT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            static_cast<int>(lc_lds(TT)));
+  if (e == hipSuccess) e = part_cu_prepare<TT, kHidSteps(kPartRanges), kPartWaves, kHidSteps(kPartRanges), false>();
+  if (e == hipSuccess) e = part_cu_prepare<TT, kInterSteps, kPartWaves, kDownBlk, false>();
+  if (e == hipSuccess) e = part_cu_prepare<TT, kHidSteps(kPartRanges), kQkvPartWaves, kHidSteps(kPartRanges), true>();
+  return e;
+}
+
+hipError_t prepare_mfma(const Dims& d) {
+  hipError_t e = hipErrorInvalidValue;
+  mf_tiles(d.batch, [&](auto tt) { e = prepare_tiles<decltype(tt)::value>(); });
   return e;
 }
 
@@ -715,7 +750,10 @@ hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, i
     a.am_bad = sc.am_bad;
     a.vocab = d.vocab;
     // one workgroup per CU; its argmax partials go straight to k_ctrl_step
-    k_mf_lm_cu<<<env.plan.argmax_parts, kLcWaves * 64, kLcLds, stream>>>(a);
+    mf_tiles(d.batch, [&](auto tt) {
+      constexpr int TT = decltype(tt)::value;
+      k_mf_lm_cu<TT><<<env.plan.argmax_parts, kLcWaves * 64, lc_lds(TT), stream>>>(a);
+    });
     return hipGetLastError();
   }
   const LayerOffsets& lo = env.layer_off[layer];
@@ -766,7 +804,10 @@ hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, i
       a.K = d.hidden;
       a.out = static_cast<bf16_t*>(sc.mlp);
       a.hidden_dim = d.intermediate;
-      k_mf_gu_cu<<<env.plan.gu_cu, kLcWaves * 64, kLcLds, stream>>>(a);
+      mf_tiles(d.batch, [&](auto tt) {
+        constexpr int TT = decltype(tt)::value;
+        k_mf_gu_cu<TT><<<env.plan.gu_cu, kLcWaves * 64, lc_lds(TT), stream>>>(a);
+      });
       break;
     case MfmaOp::kDown:
       a.x = static_cast<const bf16_t*>(sc.mlp);
