@@ -1440,9 +1440,10 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   // consumed before the next writes its own
   auto plan_of = [&](int N, int K) { return fused_mlp && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
   const GemmPlan qkv_plan = plan_of(d.qkv_rows(), d.hidden), o_plan = plan_of(d.hidden, d.q_dim()),
-                 down_plan = plan_of(d.hidden, d.intermediate);
+                 down_plan = plan_of(d.hidden, d.intermediate), kv_plan = plan_of(2 * d.kv_dim(), d.hidden);
   size_t part_bytes = 0;
-  for (const auto& [p, n] : {std::pair{qkv_plan, d.qkv_rows()}, {o_plan, d.hidden}, {down_plan, d.hidden}})
+  for (const auto& [p, n] :
+       {std::pair{qkv_plan, d.qkv_rows()}, {o_plan, d.hidden}, {down_plan, d.hidden}, {kv_plan, 2 * d.kv_dim()}})
     if (p.splits > 1) part_bytes = std::max(part_bytes, (size_t)p.splits * M * n * sizeof(float));
   const size_t o_part = fixed != nullptr ? fixed_bytes : take(part_bytes);
   if (fixed != nullptr) {
@@ -1509,7 +1510,17 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
                                    before.splits > 1 ? before.splits : 0, s));
       };
       norm(lo.input_norm, l > 0 ? down_plan : GemmPlan{4, 1});
-      gemm(o_xn, d.hidden, lo.qkv_w, lo.qkv_b, o_qkv, d.qkv_rows(), d.qkv_rows(), d.hidden, kGemmStore, qkv_plan);
+      // Nothing reads what the last layer computes past its keys and values
+      // (the first decode step starts from the prompt's last token), so it
+      // stops there: the k and v rows of the stacked projection, as a matrix
+      // of their own, and their slots.  Full model: 64 x 1,000 tokens 736.9
+      // -> 711.9 ms, four prompts of 37-250 tokens 10.87 -> 10.55; two
+      // layers of the tiny fp32 model 744 -> 606 us.
+      const bool last = l == d.layers - 1;
+      const int q_skip = last ? d.q_dim() : 0, ld = d.qkv_rows() - q_skip;
+      const GemmPlan& in_plan = last ? kv_plan : qkv_plan;
+      gemm(o_xn, d.hidden, lo.qkv_w + (size_t)q_skip * d.hidden * T, lo.qkv_b + q_skip * T, o_qkv, ld, ld, d.hidden,
+           kGemmStore, in_plan);
       PrefillQkv qp{};
       qp.qkv = b + o_qkv;
       qp.rope = er.rope;
@@ -1518,14 +1529,15 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       qp.value_cache = static_cast<uint8_t*>(e.value_cache) + l * cache_layer_elems * T;
       qp.slots = d.slots();
       qp.M = M;
-      qp.ld = d.qkv_rows();
-      qp.heads = d.heads;
+      qp.ld = ld;
+      qp.heads = last ? 0 : d.heads;
       qp.kv_heads = d.kv_heads;
       qp.head_dim = d.head_dim;
       qp.part = part;
-      qp.bias = e.weights + lo.qkv_b;
-      qp.parts = qkv_plan.splits > 1 ? qkv_plan.splits : 0;
+      qp.bias = e.weights + lo.qkv_b + q_skip * T;
+      qp.parts = in_plan.splits > 1 ? in_plan.splits : 0;
       run(launch_prefill_qkv_post(qp, d.dtype_bytes, s));
+      if (last) break;
       PrefillAttn at{};
       at.qkv = b + o_qkv;
       at.out = b + o_attn;
@@ -1558,7 +1570,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
         run(launch_prefill_swiglu(b + o_gate, b + o_up, b + o_mlp, (long long)M * d.intermediate, d.dtype_bytes, s));
       }
       gemm(o_mlp, d.intermediate, lo.down_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.intermediate, kGemmResidual,
-           down_plan);  // the last layer's residual stream is not read
+           down_plan);
     }
     if (err != hipSuccess) return -2;
   }

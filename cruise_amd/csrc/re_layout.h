@@ -290,7 +290,7 @@ struct PrefillQkv {            // RoPE in place + paged KV write
   void* key_cache;             // this layer [slots, KVH, d]
   void* value_cache;
   long long slots;
-  int M, ld, heads, kv_heads, head_dim;
+  int M, ld, heads, kv_heads, head_dim;  // heads 0: k | v rows alone
   const float* part;           // parts > 0: the rows' partial sums [parts][M][q | k | v rows] (bf16)
   const void* bias;            // T [q | k | v rows], with parts
   int parts;
