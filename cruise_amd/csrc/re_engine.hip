@@ -1427,18 +1427,14 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
     return at;
   };
   const size_t o_hidden = take(M * H * T), o_xn = take(M * H * T), o_qkv = take((size_t)M * d.qkv_rows() * T);
-  // bf16: gate, up and SwiGLU in one GEMM (no gate/up buffers); fp32: two
-  // GEMMs and the elementwise SwiGLU
-  const bool fused_mlp = d.dtype_bytes == 2;
-  const size_t o_attn = take((size_t)M * d.q_dim() * T), o_gate = fused_mlp ? 0 : take(M * I * T);
-  const size_t o_up = fused_mlp ? 0 : take(M * I * T);
+  const size_t o_attn = take((size_t)M * d.q_dim() * T);
   const size_t o_mlp = take(M * I * T), o_rope = take((size_t)M * d.head_dim * sizeof(float));
   const size_t o_tok = take(8 * (size_t)M), o_pos = take(4 * (size_t)M), o_slot = take(4 * (size_t)M);
   const size_t o_tiles = take(sizeof(int4) * tiles.size()), o_blocks = take(4 * tables.size());
   const size_t rows_bytes = off;
   // K ranges of the qkv, o and down GEMMs (bf16); each one's partial sums are
   // consumed before the next writes its own
-  auto plan_of = [&](int N, int K) { return fused_mlp && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
+  auto plan_of = [&](int N, int K) { return T == 2 && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
   const GemmPlan qkv_plan = plan_of(d.qkv_rows(), d.hidden), o_plan = plan_of(d.hidden, d.q_dim()),
                  down_plan = plan_of(d.hidden, d.intermediate), kv_plan = plan_of(2 * d.kv_dim(), d.hidden);
   size_t part_bytes = 0;
@@ -1551,24 +1547,18 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       run(launch_prefill_attention(at, d, static_cast<int>(tiles.size()), s));
       gemm(o_attn, d.q_dim(), lo.o_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.q_dim(), kGemmResidual, o_plan);
       norm(lo.post_norm, o_plan);
-      if (fused_mlp) {
-        GemmArgs g{};
-        g.A = b + o_xn;
-        g.W = e.weights + lo.gate_w;
-        g.W2 = e.weights + lo.up_w;
-        g.out = b + o_mlp;
-        g.M = M;
-        g.N = d.intermediate;
-        g.K = d.hidden;
-        g.lda = d.hidden;
-        g.ldw = d.hidden;
-        g.ldo = d.intermediate;
-        run(launch_gemm(g, kGemmSwiGlu, d.dtype_bytes, s));
-      } else {
-        gemm(o_xn, d.hidden, lo.gate_w, SIZE_MAX, o_gate, d.intermediate, d.intermediate, d.hidden, kGemmStore);
-        gemm(o_xn, d.hidden, lo.up_w, SIZE_MAX, o_up, d.intermediate, d.intermediate, d.hidden, kGemmStore);
-        run(launch_prefill_swiglu(b + o_gate, b + o_up, b + o_mlp, (long long)M * d.intermediate, d.dtype_bytes, s));
-      }
+      GemmArgs gu{};
+      gu.A = b + o_xn;
+      gu.W = e.weights + lo.gate_w;
+      gu.W2 = e.weights + lo.up_w;
+      gu.out = b + o_mlp;
+      gu.M = M;
+      gu.N = d.intermediate;
+      gu.K = d.hidden;
+      gu.lda = d.hidden;
+      gu.ldw = d.hidden;
+      gu.ldo = d.intermediate;
+      run(launch_gemm(gu, kGemmSwiGlu, d.dtype_bytes, s));
       gemm(o_mlp, d.intermediate, lo.down_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.intermediate, kGemmResidual,
            down_plan);
     }
@@ -1873,7 +1863,8 @@ extern "C" int32_t resident_epoch_gemm(const void* A, const void* W, const void*
                                        int32_t M, int32_t N, int32_t K, int32_t epilogue, int32_t dtype_bytes) {
   using namespace re;
   if (A == nullptr || W == nullptr || out == nullptr || M < 0 || N <= 0 || K <= 0 || epilogue < kGemmStore ||
-      epilogue > kGemmSwiGlu || (dtype_bytes != 2 && dtype_bytes != 4) || (epilogue == kGemmSwiGlu && W2 == nullptr))
+      epilogue > kGemmSwiGlu || (dtype_bytes != 2 && dtype_bytes != 4) ||
+      (epilogue == kGemmSwiGlu && (W2 == nullptr || dtype_bytes != 2)))
     return -1;
   // the bf16 kernel reads the bias four elements at a time
   if (dtype_bytes == 2 && epilogue == kGemmStore && bias != nullptr && (reinterpret_cast<uintptr_t>(bias) & 7) != 0)

@@ -302,8 +302,8 @@ struct PrefillAttn {           // causal attention within each row's prompt
   const int4* tiles;           // MFMA path: {first query token, row's first token, queries, first position}
   int M, ld, heads, kv_heads, head_dim;
 };
-// Store: out = T(acc + bias); Residual: out = T(out + T(acc)); SwiGlu (bf16
-// only): W holds the gate rows and W2 the up rows, and out[m, n] =
+// Store: out = T(acc + bias); Residual: out = T(out + T(acc)); SwiGlu: W holds
+// the gate rows and W2 the up rows, and out[m, n] =
 // T(T(silu(T(gate))) * T(up)) over N output columns.
 // Part (bf16 only): the fp32 partial sums of K ranges, to part.
 enum GemmEpilogue : int { kGemmStore = 0, kGemmResidual = 1, kGemmSwiGlu = 2, kGemmPart = 3 };
@@ -325,8 +325,6 @@ hipError_t launch_prefill_embed(const PrefillRows& a, int dtype_bytes, hipStream
 // parts > 0: x += the partial sums [parts][M][H] of a split GEMM first (bf16).
 hipError_t launch_prefill_rmsnorm(void* x, const void* w, void* y, int M, int H, float eps, int dtype_bytes,
                                   const float* part, int parts, hipStream_t stream);
-hipError_t launch_prefill_swiglu(const void* gate, const void* up, void* out, long long n, int dtype_bytes,
-                                 hipStream_t stream);
 hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStream_t stream);
 // The fastest tile and K ranges for a shape whose partial sums take at most
 // part_bytes; launch_gemm follows `plan` when a.part is set, else it picks the

@@ -12,16 +12,15 @@
 //              "T(h + T(acc))", and gate/up with SwiGLU in one GEMM (the
 //              tile's W rows half gate, half up); K split over workgroups
 //              where the tiles alone leave CUs idle, the partial sums added
-//              by the row kernel that follows.  fp32 models: an LDS-tiled
-//              FMA GEMM.
+//              by the row kernel that follows.  fp32 models: 16 x 16 and
+//              32 x 32 tiles on the fp32 MFMA, K split over a workgroup's
+//              waves, the same epilogues.
 //   qkv post   RoPE of q and k in place, K/V rows to their paged slots
 //   attention  causal within each row's prompt.  bf16, head_dim 128: MFMA
 //              for Q K^T and P V per (64-query tile, head), the bf16 scores of
 //              the whole tile kept in LDS so the softmax is the exact
 //              two-pass one of the decode step; otherwise one workgroup per
 //              (token, head).
-//   SwiGLU     elementwise on the gate and up products (fp32 models; bf16
-//              models take it in the gate/up GEMM's epilogue)
 #include <algorithm>
 #include <type_traits>
 
@@ -145,29 +144,6 @@ __global__ void __launch_bounds__(PART ? 512 : 256) k_pf_rmsnorm(void* x, const 
 #pragma unroll
     for (int e = 0; e < 8; ++e) out[e] = Elt<T>::r(Elt<T>::r(v[i].get(e) * rs) * g.get(e));
     *reinterpret_cast<Vec8<T>*>(yr + c * 8) = Vec8<T>::from_floats(out);
-  }
-}
-
-// gate = silu(g), product with up (batched_decoder_step.py:391-398); g and up
-// arrive rounded to T by their GEMMs.
-// Eight elements per thread and step (16-byte bf16 accesses); n % 8 == 0.
-template <typename T>
-__global__ void __launch_bounds__(256) k_pf_swiglu(const void* gate, const void* up, void* out, long long n) {
-  const T* g = static_cast<const T*>(gate);
-  const T* u = static_cast<const T*>(up);
-  T* o = static_cast<T*>(out);
-  const long long nv = n / 8;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += (long long)gridDim.x * blockDim.x) {
-    const Vec8<T> gv = Vec8<T>::load(g + i * 8);
-    const Vec8<T> uv = Vec8<T>::load(u + i * 8);
-    float y[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = gv.get(e);
-      const float sg = Elt<T>::r(x / (1.0f + expf(-x)));
-      y[e] = Elt<T>::r(sg * uv.get(e));
-    }
-    *reinterpret_cast<Vec8<T>*>(o + i * 8) = Vec8<T>::from_floats(y);
   }
 }
 
@@ -591,56 +567,114 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   }
 }
 
-// fp32 models: 64 x 64 tiles, 4 x 4 outputs per thread, K in steps of 16.
-template <int EPI>
-__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Ws[16][64 + 4];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const float* A = static_cast<const float*>(a.A);
-  const float* W = static_cast<const float*>(a.W);
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < a.K; k0 += 16) {
+// fp32 models: one 16 MT x 16 MT output tile per workgroup of four waves, on
+// v_mfma_f32_16x16x4_f32 (fp32 operands and sums).  K goes to the waves in
+// 16-element chunks, chunk c to wave c % 4, so the workgroup reads its rows in
+// contiguous 256-byte pieces; a lane takes four consecutive K elements of its
+// row of each operand straight from memory (16 bytes), and instruction e of a
+// chunk multiplies element e of every lane: its four k indexes are elements
+// e, 4 + e, 8 + e and 12 + e of the chunk, in both operands alike.  As in the
+// bf16 kernel the products run as C^T = W A^T.  The four waves' sums are added
+// in wave order through LDS.  K need not be a multiple of anything and the
+// operands need no alignment past 4 bytes: VEC = false loads element by
+// element.
+//
+// What bounds it: the products are small (the tiny test model: 66 tokens,
+// K = 256 and 688), so latency does: one chain of loads per K chunk.  The
+// chunks are spread over four waves and UN of them are in flight at once, and
+// the tile is 16 x 16 while 32 x 32 would not give every CU two workgroups.
+// 66 tokens, before (64 x 64 tiles through LDS on the vector units) and now:
+// K = 256, N = 512 24.2 -> 3.8 us; K = 688, N = 256 63.7 -> 5.0 us.
+//
+// SwiGLU: W the gate rows, W2 the up rows, out = silu(gate) * up.
+template <int EPI, int MT, bool VEC>
+__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN) {
+  constexpr int kT = 16 * MT, kOps = EPI == kGemmSwiGlu ? 2 : 1, kLd = kT + 4;
+  constexpr int UN = MT == 1 ? 4 : 2;
+  __shared__ __align__(16) float red[4][kOps][kT][kLd];
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
+  const int m0 = blockIdx.x / nN * kT, n0 = blockIdx.x % nN * kT;
+  const int fr = lane & 15, fq = lane >> 4;
+  // Rows past M or N read a valid row (clamped) whose results are never stored.
+  const float* arow[MT];
+  const float* wrow[kOps][MT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = tid + 256 * i, row = idx >> 4, kk = idx & 15, k = k0 + kk;
-      const bool kin = k < a.K;
-      const float x = A[(size_t)min(m0 + row, a.M - 1) * a.lda + (kin ? k : 0)];
-      const float y = W[(size_t)min(n0 + row, a.N - 1) * a.ldw + (kin ? k : 0)];
-      As[kk][row] = kin ? x : 0.f;
-      Ws[kk][row] = kin ? y : 0.f;
-    }
-    __syncthreads();
+  for (int j = 0; j < MT; ++j) {
+    arow[j] = static_cast<const float*>(a.A) + (size_t)min(m0 + 16 * j + fr, a.M - 1) * a.lda;
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float av[4], wv[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        av[r] = As[kk][ty * 4 + r];
-        wv[r] = Ws[kk][tx * 4 + r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] = fmaf(av[r], wv[c], acc[r][c]);
-    }
-    __syncthreads();
+    for (int b = 0; b < kOps; ++b)
+      wrow[b][j] = static_cast<const float*>(b == 0 ? a.W : a.W2) + (size_t)min(n0 + 16 * j + fr, a.N - 1) * a.ldw;
   }
+  // four elements of a row from k on; zero past K
+  auto load4 = [&](const float* row, int k) -> f32x4_t {
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (VEC) {
+      if (k < a.K) v = *reinterpret_cast<const f32x4_t*>(row + k);  // K % 4 == 0
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (k + e < a.K) v[e] = row[k + e];
+    }
+    return v;
+  };
+  f32x4_t acc[kOps][MT][MT];  // [operand][n][m]
+#pragma unroll
+  for (int b = 0; b < kOps; ++b)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[b][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = wave * 16; k0 < a.K; k0 += 64 * UN) {
+    f32x4_t av[UN][MT], wv[UN][kOps][MT];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int k = k0 + 64 * u + 4 * fq;
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        av[u][j] = load4(arow[j], k);
+#pragma unroll
+        for (int b = 0; b < kOps; ++b) wv[u][b][j] = load4(wrow[b][j], k);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int b = 0; b < kOps; ++b)
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+              acc[b][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][b][i][e], av[u][j][e], acc[b][i][j], 0, 0, 0);
+  }
+  // acc value v of lane l: n = 4 (l / 16) + v, m = l % 16 within its 16 x 16 block
+#pragma unroll
+  for (int b = 0; b < kOps; ++b)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        *reinterpret_cast<f32x4_t*>(&red[wave][b][16 * j + fr][16 * i + 4 * fq]) = acc[b][i][j];
+  __syncthreads();
   float* out = static_cast<float*>(a.out);
   const float* bias = static_cast<const float*>(a.bias);
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int idx = tid; idx < kT * kT; idx += 256) {
+    const int ml = idx / kT, nl = idx % kT, m = m0 + ml, n = n0 + nl;
+    if (m >= a.M || n >= a.N) continue;
+    float y[kOps];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int m = m0 + ty * 4 + r, n = n0 + tx * 4 + c;
-      if (m >= a.M || n >= a.N) continue;
-      float* o = out + (size_t)m * a.ldo + n;
-      if constexpr (EPI == kGemmStore)
-        *o = acc[r][c] + (bias != nullptr ? bias[n] : 0.f);
-      else
-        *o = *o + acc[r][c];
-    }
+    for (int b = 0; b < kOps; ++b)
+      y[b] = ((red[0][b][ml][nl] + red[1][b][ml][nl]) + red[2][b][ml][nl]) + red[3][b][ml][nl];
+    float* o = out + (size_t)m * a.ldo + n;
+    if constexpr (EPI == kGemmStore)
+      *o = y[0] + (bias != nullptr ? bias[n] : 0.f);
+    else if constexpr (EPI == kGemmResidual)
+      *o = *o + y[0];
+    else
+      *o = y[0] / (1.0f + expf(-y[0])) * y[kOps - 1];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -998,18 +1032,6 @@ hipError_t launch_prefill_rmsnorm(void* x, const void* w, void* y, int M, int H,
   return hipGetLastError();
 }
 
-hipError_t launch_prefill_swiglu(const void* gate, const void* up, void* out, long long n, int dtype_bytes,
-                                 hipStream_t stream) {
-  if (n <= 0) return hipSuccess;
-  if (n % 8 != 0) return hipErrorInvalidValue;  // rows of the intermediate size, a multiple of 8
-  const int blocks = static_cast<int>(std::min<long long>((n / 8 + 255) / 256, 16384));
-  if (dtype_bytes == 2)
-    k_pf_swiglu<bf16_t><<<blocks, 256, 0, stream>>>(gate, up, out, n);
-  else
-    k_pf_swiglu<float><<<blocks, 256, 0, stream>>>(gate, up, out, n);
-  return hipGetLastError();
-}
-
 hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStream_t stream) {
   if (a.M <= 0) return hipSuccess;
   if (a.head_dim % 16 != 0 || a.ld % 8 != 0) return hipErrorInvalidValue;
@@ -1044,6 +1066,32 @@ static hipError_t gemm_launch_mj(const GemmArgs& a, const GemmPlan& p, hipStream
     case 3: return gemm_launch<EPI, 3>(a, p.splits, stream);
     default: return gemm_launch<EPI, 4>(a, p.splits, stream);
   }
+}
+
+// 32 x 32 tiles (twice the products per byte) where they still are two
+// workgroups per CU, else 16 x 16.  Both measured (M x N x K, 16 x 16 against
+// 32 x 32): 66 x 256 x 688 5.0 and 8.9 us, 500 x 256 x 688 6.8 and 9.2, 500 x
+// 512 x 256 6.7 and 6.0; 2,044 x 256 x 688 20.0 and 15.6, 2,044 x 1,376 x 256
+// 44.0 and 31.2, 8,000 x 512 x 256 61.2 and 43.1.
+template <int EPI>
+static hipError_t gemm_f32_launch(const GemmArgs& a, hipStream_t stream) {
+  constexpr long long kLargeTiles = 2 * 256;
+  auto tiles = [&](int t) { return (long long)((a.M + t - 1) / t) * ((a.N + t - 1) / t); };
+  const bool large = tiles(32) >= kLargeTiles;
+  const long long grid = tiles(large ? 32 : 16);
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  const int nN = (a.N + (large ? 31 : 15)) / (large ? 32 : 16);
+  const uintptr_t addr = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W) |
+                         (EPI == kGemmSwiGlu ? reinterpret_cast<uintptr_t>(a.W2) : 0);
+  const bool vec = (addr & 15) == 0 && a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0;
+  auto run = [&](auto mt, auto v) {
+    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<static_cast<unsigned>(grid), 256, 0, stream>>>(a, nN);
+    return hipGetLastError();
+  };
+  using one = std::integral_constant<int, 1>;
+  using two = std::integral_constant<int, 2>;
+  if (large) return vec ? run(two{}, std::true_type{}) : run(two{}, std::false_type{});
+  return vec ? run(one{}, std::true_type{}) : run(one{}, std::false_type{});
 }
 
 // Tile height and K ranges of a bf16 GEMM: the pair with the least estimated
@@ -1097,14 +1145,11 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t 
     if (epi == kGemmResidual) return gemm_launch_mj<kGemmResidual>(a, p, stream);
     return gemm_launch_mj<kGemmSwiGlu>(a, p, stream);
   } else {
-    if (a.K <= 0 || epi == kGemmSwiGlu || a.part != nullptr) return hipErrorInvalidValue;
-    const dim3 grid((a.N + 63) / 64, (a.M + 63) / 64);
-    if (epi == kGemmStore)
-      k_gemm_f32<kGemmStore><<<grid, 256, 0, stream>>>(a);
-    else
-      k_gemm_f32<kGemmResidual><<<grid, 256, 0, stream>>>(a);
+    if (a.K <= 0 || a.part != nullptr || (epi == kGemmSwiGlu && a.W2 == nullptr)) return hipErrorInvalidValue;
+    if (epi == kGemmStore) return gemm_f32_launch<kGemmStore>(a, stream);
+    if (epi == kGemmResidual) return gemm_f32_launch<kGemmResidual>(a, stream);
+    return gemm_f32_launch<kGemmSwiGlu>(a, stream);
   }
-  return hipGetLastError();
 }
 
 // The MFMA attention serves bf16 models with head_dim 128 (any window: its
