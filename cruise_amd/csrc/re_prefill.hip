@@ -239,14 +239,14 @@ __global__ void __launch_bounds__(PART ? 512 : 256) k_pf_qkv_post(PrefillQkv a) 
 // Chunk c (16 bytes) of row r sits in slot c ^ gemm_swz(r), so the fragment
 // reads below hit distinct banks for 8 and for 16 consecutive rows.  The
 // products run as C^T = W A^T on v_mfma_f32_16x16x32_bf16: wave (wn, wm) owns
-// n 128 x m 16 MJ (8 x MJ tiles of 16 x 16), and a lane's accumulator holds four
-// consecutive output columns of one row.  A stage is two sub-steps of K = 32;
-// each sub-step's 8 + MJ fragments are read under the previous sub-step's 8 MJ
-// products.  The stage's one barrier sits between its sub-steps: before it
+// NI x MI tiles of 16 x 16 (n x m, gemm_waves_n), and a lane's accumulator holds
+// four consecutive output columns of one row.  A stage is two sub-steps of K =
+// 32; each sub-step's NI + MI fragments are read under the previous sub-step's
+// NI MI products.  The stage's one barrier sits between its sub-steps: before it
 // each wave waits for its own loads of stage kt + 1 and its reads of stage
 // kt, so after it stage kt + 1 is complete in LDS and stage kt's buffer is
 // free.  The loads of stage kt + ST go out during the second sub-step (waves
-// 0-3 at its start, waves 4-7 after 3 of their 8 row blocks, so the two waves
+// 0-3 at its start, waves 4-7 after 3/8 of their products, so the two waves
 // of a SIMD do not stall on them together), and stage kt + 1's first
 // fragments are read under the second sub-step's products, so no wave waits
 // on LDS at a stage boundary.  The epilogue rounds the tile to bf16 in LDS
@@ -265,7 +265,10 @@ __global__ void __launch_bounds__(PART ? 512 : 256) k_pf_qkv_post(PrefillQkv a) 
 // tile t = (b % 8) * ceil(T / 8) + b / 8 of an order with the K ranges
 // outermost and the tiles of a range grouped (4 M tiles by every N tile), so
 // the 32 tiles an XCD runs at once share 4 A and 8 W row blocks in its L2,
-// and the tiles of a K range share its columns of A.
+// and the tiles of a K range share its columns of A.  Up to 8 M tiles are one
+// group, so W is read through once (gate/up at 400 tokens, 64-row tiles: 210
+// -> 186 us in one group of 7 instead of groups of 4 and 3; at 570 and 1,000
+// tokens, 128-row tiles, 171.6 -> 169.7 and 281.8 -> 278.0).
 //
 // Requirements (checked by launch_gemm): K % 64 == 0, N % 8 == 0, lda, ldw
 // and ldo multiples of 8 elements, 16-byte aligned operands.
@@ -309,17 +312,26 @@ __device__ __forceinline__ void gemm_tile_of(int b, int nM, int nN, int nS, int&
   int t = x < r ? x * (q + 1) + local : r * (q + 1) + (x - r) * q + local;
   ks = t / tiles;
   t -= ks * tiles;
-  const int per_group = kGgroupM * nN, g = t / per_group, first = g * kGgroupM;
-  const int gm = min(kGgroupM, nM - first), w = t - g * per_group;
+  const int group_m = nM <= 2 * kGgroupM ? nM : kGgroupM;
+  const int per_group = group_m * nN, g = t / per_group, first = g * group_m;
+  const int gm = min(group_m, nM - first), w = t - g * per_group;
   mt = first + w % gm;
   nt = w / gm;
 }
 
+// Waves along n: a wave's block of 16 x 16 tiles is 8 x 4 (n x m) of a 256-row
+// tile and 4 x 6, 4 x 4 and 4 x 2 of the lower ones, the fewest fragment reads
+// per product (two waves along n throughout: 11 reads for 24 products, 10 for
+// 16 and 9 for 8 instead of 10, 8 and 6).  Gate/up at 570 tokens, 128-row tiles:
+// 181 -> 171 us; 400 tokens 170 -> 161; 2,000 tokens, 64-row tiles 811 -> 774;
+// 192-row tiles the same within 1 %.
+constexpr int gemm_waves_n(int mj) { return mj == 4 ? 2 : 4; }
+
 // Fragments of the next stage read before product p of the second sub-step:
 // one per two products where that covers them, else spread over the first 7/8
 // of the products.
-constexpr int gemm_reads_by(int mj, int p) {
-  const int frags = 8 + mj, prods = 8 * mj, span = prods - prods / 8;
+constexpr int gemm_reads_by(int frags, int prods, int p) {
+  const int span = prods - prods / 8;
   const int n = 2 * frags <= prods ? p / 2 : (p * frags + span - 1) / span;
   return n < frags ? n : frags;
 }
@@ -399,12 +411,13 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
                                          (gemm_lptr)(l + lrow[1] * kGrowBytes + (i - 4) * 1024), 16, 0, 0);
     }
   };
-  const int wn = wave & 1, wm = wave >> 1;
-  f32x4_t acc[8][MJ];
+  constexpr int kWn = gemm_waves_n(MJ), NI = 16 / kWn, MI = 4 * MJ / (kGwaves / kWn);
+  const int wn = wave % kWn, wm = wave / kWn;
+  f32x4_t acc[NI][MI];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < MJ; ++j)
+    for (int j = 0; j < MI; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
   // lane l supplies row l % 16 of a 16-row operand tile, K elements
@@ -415,11 +428,11 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   auto frag = [&](int st, int row0, int ks2) -> bf16x8_t {
     return lds_frag(reinterpret_cast<const bf16_t*>(gsm + st * kStage + row0 * kGrowBytes + frag_off[ks2]));
   };
-  // fragment sets: [set][0..7] W rows (n), [set][8..] A rows (m)
-  constexpr int kFrags = 8 + MJ, kProds = 8 * MJ;
+  // fragment sets: [set][0 .. NI - 1] W rows (n), [set][NI ..] A rows (m)
+  constexpr int kFrags = NI + MI, kProds = NI * MI;
   bf16x8_t f[2][kFrags];
   auto read_frag = [&](int set, int idx, int st, int ks2) {
-    f[set][idx] = idx < 8 ? frag(st, wn * 128 + idx * 16, ks2) : frag(st, kGn + wm * 16 * MJ + (idx - 8) * 16, ks2);
+    f[set][idx] = idx < NI ? frag(st, (wn * NI + idx) * 16, ks2) : frag(st, kGn + (wm * MI + idx - NI) * 16, ks2);
   };
   auto read_set = [&](int set, int st, int ks2) {
 #pragma unroll
@@ -427,10 +440,10 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   };
   auto products = [&](int set) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < MJ; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[set][i], f[set][8 + j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < MI; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[set][i], f[set][NI + j], acc[i][j], 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < kFrags; ++r) {  // fragment reads spread over the products
       __builtin_amdgcn_sched_group_barrier(0x008, kProds / kFrags > 0 ? kProds / kFrags : 1, 0);
@@ -473,17 +486,15 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
     // waits while the memory pipeline takes its 1 KB requests, and meanwhile
     // the other wave's products run.
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i == 0 && wave < 4 && more) issue(next, st);
-      if (i == 3 && wave >= 4 && more) issue(next, st);
+    for (int p = 0; p < kProds; ++p) {
+      const int i = p / MI, j = p % MI;
+      if (p == 0 && wave < 4 && more) issue(next, st);
+      if (p == kProds * 3 / 8 && wave >= 4 && more) issue(next, st);
+      if (j == 0) __builtin_amdgcn_sched_barrier(0);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][i], f[1][NI + j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int r = gemm_reads_by(kFrags, kProds, p); r < gemm_reads_by(kFrags, kProds, p + 1); ++r) read_frag(0, r, nst, 0);
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][i], f[1][8 + j], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int r = gemm_reads_by(MJ, i * MJ + j); r < gemm_reads_by(MJ, i * MJ + j + 1); ++r) read_frag(0, r, nst, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
     }
     ring = nst;
   }
@@ -492,10 +503,10 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   if constexpr (kPart) {
     // fp32 partial sums [nS][M][N], four consecutive columns per lane
 #pragma unroll
-    for (int j = 0; j < MJ; ++j)
+    for (int j = 0; j < MI; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int m = m0 + wm * 16 * MJ + j * 16 + fr, n = n0 + wn * 128 + i * 16 + 4 * fq;
+      for (int i = 0; i < NI; ++i) {
+        const int m = m0 + (wm * MI + j) * 16 + fr, n = n0 + (wn * NI + i) * 16 + 4 * fq;
         if (m < a.M && n < a.N)
           *reinterpret_cast<f32x4_t*>(a.part + ((size_t)ks * a.M + m) * a.N + n) = acc[i][j];
       }
@@ -505,10 +516,10 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   bf16_t* T = reinterpret_cast<bf16_t*>(gsm);
   const bf16_t* bias = static_cast<const bf16_t*>(a.bias);
 #pragma unroll
-  for (int j = 0; j < MJ; ++j)
+  for (int j = 0; j < MI; ++j)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int ml = wm * 16 * MJ + j * 16 + fr, nl = wn * 128 + i * 16 + 4 * fq;
+    for (int i = 0; i < NI; ++i) {
+      const int ml = (wm * MI + j) * 16 + fr, nl = (wn * NI + i) * 16 + 4 * fq;
       float y[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = acc[i][j][e];
