@@ -780,6 +780,26 @@ hipError_t launch_clear_blocks(const KernelEnv& env, void* key_cache, void* valu
   return hipGetLastError();
 }
 
+namespace {
+// One thread per row (at most 256).
+__global__ void __launch_bounds__(256) k_store_rows(StatePtrs s, const RowRecord* rows, int n) {
+  const int i = threadIdx.x;
+  if (i >= n) return;
+  const RowRecord r = rows[i];
+  s.res_gen[r.row] = r.generation;
+  s.res_token[r.row] = r.token;
+  s.res_pos[r.row] = r.length - 1;
+  s.res_len[r.row] = r.length;
+  s.res_valid[r.row] = 1;
+}
+}  // namespace
+
+hipError_t launch_store_rows(const StatePtrs& st, const RowRecord* rows, int n, hipStream_t stream) {
+  if (n < 0 || n > 256) return hipErrorInvalidValue;
+  k_store_rows<<<1, 256, 0, stream>>>(st, rows, n);
+  return hipGetLastError();
+}
+
 hipError_t launch_fill_synthetic(void* dst, long long elems, int dtype_bytes, unsigned long long seed,
                                  unsigned long long stream_id, float std_dev, hipStream_t stream) {
   k_fill_normal<<<4096, 256, 0, stream>>>(dst, elems, dtype_bytes, seed, stream_id, std_dev);

@@ -136,6 +136,7 @@ struct Engine {
 
   // decoder-step ABI buffers
   uint8_t* step_mem = nullptr;
+  size_t step_in_bytes = 0;  // its inputs, next_pos behind them
   StepPtrs step_io{};
   void* dec_key = nullptr;
   void* dec_value = nullptr;
@@ -143,6 +144,7 @@ struct Engine {
   // host staging (pinned)
   uint8_t* h_feed = nullptr;
   uint8_t* h_fetch = nullptr;
+  uint8_t* h_step = nullptr;  // the step inputs, laid out as in step_mem
   size_t feed_bytes = 0, import_feed_bytes = 0, fetch_bytes = 0, payload_bytes = 0;
   // Batched prefill scratch (grown on demand, freed with the engine).
   uint8_t* pf_mem = nullptr;
@@ -554,6 +556,7 @@ bool alloc_state(Engine& e) {
     offs.push_back(off);
     off = align_up(off + pr.bytes, 256);
   }
+  e.step_in_bytes = offs.back();
   if (hipMalloc(&e.step_mem, off) != hipSuccess) return false;
   if (hipMemset(e.step_mem, 0, off) != hipSuccess) return false;
   for (size_t i = 0; i < io.size(); ++i) *io[i].p = e.step_mem + offs[i];
@@ -577,6 +580,8 @@ bool alloc_state(Engine& e) {
   if (hipHostMalloc(reinterpret_cast<void**>(&e.h_feed), align_up(e.import_feed_bytes, 4096), 0) != hipSuccess)
     return false;
   if (hipHostMalloc(reinterpret_cast<void**>(&e.h_fetch), align_up(e.fetch_bytes, 4096), 0) != hipSuccess)
+    return false;
+  if (hipHostMalloc(reinterpret_cast<void**>(&e.h_step), align_up(e.step_in_bytes, 4096), 0) != hipSuccess)
     return false;
   std::memset(e.h_feed, 0, e.import_feed_bytes);
   std::memset(e.h_fetch, 0, e.fetch_bytes);
@@ -783,6 +788,7 @@ void free_state(Engine& e) {
   drop(e.step_mem);
   drop_host(e.h_feed);
   drop_host(e.h_fetch);
+  drop_host(e.h_step);
 }
 
 void free_engine(Engine* e) {
@@ -1270,11 +1276,57 @@ extern "C" int32_t resident_epoch_proc(void* engine, const void* feed, int64_t f
 }
 
 namespace {
-bool copy_in(void* dst, const void* src, size_t bytes, hipStream_t s) {
-  return hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, s) == hipSuccess;
+// Memory the host can read and write itself (pageable or pinned).
+bool host_memory(const void* p) {
+  hipPointerAttribute_t attr{};
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return attr.type == hipMemoryTypeUnregistered || attr.type == hipMemoryTypeHost;
+}
+
+// Device memory of `device` that holds bytes from p on, aligned for the kernels.
+bool device_memory(void* p, size_t bytes, int device) {
+  hipPointerAttribute_t attr{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess || attr.type != hipMemoryTypeDevice || attr.device != device ||
+      hipMemGetAddressRange(&base, &size, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const size_t at = static_cast<uint8_t*>(p) - static_cast<uint8_t*>(base);
+  return reinterpret_cast<uintptr_t>(p) % 16 == 0 && at <= size && bytes <= size - at;
+}
+
+// Where a step input goes in the pinned staging copy of step_mem.
+template <typename P>
+P* staged(re::Engine& e, const P* dev) {
+  return reinterpret_cast<P*>(e.h_step + (reinterpret_cast<const uint8_t*>(dev) - e.step_mem));
+}
+
+bool upload_step(re::Engine& e) {
+  return hipMemcpyAsync(e.step_mem, e.h_step, e.step_in_bytes, hipMemcpyHostToDevice, e.stream) == hipSuccess;
+}
+
+// Resident records of rows, written on the engine's stream after what is
+// queued there; the caller waits for the stream.
+bool store_rows(re::Engine& e, const std::vector<re::RowRecord>& rows) {
+  const size_t bytes = rows.size() * sizeof(re::RowRecord);
+  static_assert(sizeof(re::RowRecord) <= 28, "a feed holds at least 28 bytes a row");
+  std::memcpy(e.h_feed, rows.data(), bytes);
+  return hipMemcpyAsync(e.st.feed, e.h_feed, bytes, hipMemcpyHostToDevice, e.stream) == hipSuccess &&
+         re::launch_store_rows(e.st, reinterpret_cast<const re::RowRecord*>(e.st.feed), static_cast<int>(rows.size()),
+                               e.stream) == hipSuccess;
 }
 }  // namespace
 
+// What a step takes beyond its kernels is copies and waits, so: inputs in host
+// memory go up in one pinned copy, caches in this device's memory are used in
+// place (others go through the engine's own pair), next_position comes from the
+// embedding kernel, and there is one wait.  One layer and the head, four rows:
+// 379 -> 307 us.
 extern "C" int32_t resident_decoder_step(void* engine, const int64_t* token_id, const int64_t* position,
                                          const int32_t* sequence_length, void* key_cache,
                                          const int32_t* slot_mapping, const int32_t* active_mask,
@@ -1290,37 +1342,52 @@ extern "C" int32_t resident_decoder_step(void* engine, const int64_t* token_id, 
   const Dims& d = e->dims;
   const int B = d.batch;
   hipStream_t s = e->stream;
-  if (e->dec_key == nullptr) {
+  const size_t cache_gap = key_cache < value_cache
+                               ? static_cast<uint8_t*>(value_cache) - static_cast<uint8_t*>(key_cache)
+                               : static_cast<uint8_t*>(key_cache) - static_cast<uint8_t*>(value_cache);
+  const bool in_place = cache_gap >= e->cache_bytes && device_memory(key_cache, e->cache_bytes, e->device) &&
+                        device_memory(value_cache, e->cache_bytes, e->device);
+  if (!in_place && e->dec_key == nullptr) {
     if (hipMalloc(&e->dec_key, e->cache_bytes) != hipSuccess) return -2;
     if (hipMalloc(&e->dec_value, e->cache_bytes) != hipSuccess) return -2;
   }
   StepPtrs sp = e->step_io;
-  bool ok = copy_in(const_cast<int64_t*>(sp.token), token_id, 8 * B, s) &&
-            copy_in(const_cast<int64_t*>(sp.pos), position, 8 * B, s) &&
-            copy_in(const_cast<int32_t*>(sp.len), sequence_length, 4 * B, s) &&
-            copy_in(const_cast<int32_t*>(sp.slot), slot_mapping, 4 * B, s) &&
-            copy_in(const_cast<int32_t*>(sp.active), active_mask, 4 * B, s) &&
-            copy_in(const_cast<int32_t*>(sp.table), block_table, 4 * (size_t)B * d.blocks_per_row, s) &&
-            copy_in(e->dec_key, key_cache, e->cache_bytes, s) && copy_in(e->dec_value, value_cache, e->cache_bytes, s);
-  if (!ok) return -2;
-  sp.key_cache = e->dec_key;
-  sp.value_cache = e->dec_value;
+  struct Input {
+    const void* dev;
+    const void* src;
+    size_t bytes;
+    bool host;
+  };
+  Input inputs[] = {{sp.token, token_id, 8 * (size_t)B, true},
+                    {sp.pos, position, 8 * (size_t)B, true},
+                    {sp.len, sequence_length, 4 * (size_t)B, true},
+                    {sp.slot, slot_mapping, 4 * (size_t)B, true},
+                    {sp.active, active_mask, 4 * (size_t)B, true},
+                    {sp.table, block_table, 4 * (size_t)B * d.blocks_per_row, true}};
+  bool any_host = false;
+  for (Input& in : inputs) {
+    in.host = host_memory(in.src);
+    any_host |= in.host;
+    if (in.host) std::memcpy(staged(*e, static_cast<const uint8_t*>(in.dev)), in.src, in.bytes);
+  }
+  sp.key_cache = in_place ? key_cache : e->dec_key;
+  sp.value_cache = in_place ? value_cache : e->dec_value;
   sp.logits = e->logits;
   sp.done = nullptr;
-  if (launch_decoder_step(e->env(), sp, s) != hipSuccess) return -2;
-  std::vector<int64_t> pos(B), npos(B);
-  std::vector<int32_t> act(B);
-  ok = hipMemcpyAsync(pos.data(), sp.pos, 8 * B, hipMemcpyDeviceToHost, s) == hipSuccess &&
-       hipMemcpyAsync(act.data(), sp.active, 4 * B, hipMemcpyDeviceToHost, s) == hipSuccess &&
-       hipMemcpyAsync(logits, e->logits, (size_t)B * d.vocab * sizeof(float), hipMemcpyDefault, s) == hipSuccess &&
-       hipMemcpyAsync(key_cache, e->dec_key, e->cache_bytes, hipMemcpyDefault, s) == hipSuccess &&
-       hipMemcpyAsync(value_cache, e->dec_value, e->cache_bytes, hipMemcpyDefault, s) == hipSuccess &&
-       hipStreamSynchronize(s) == hipSuccess;
-  if (!ok) return -2;
-  // next_position = where(active, pos + 1, pos) (batched_decoder_step.py:409-411)
-  for (int b = 0; b < B; ++b) npos[b] = act[b] != 0 ? pos[b] + 1 : pos[b];
-  if (hipMemcpy(next_position, npos.data(), 8 * B, hipMemcpyDefault) != hipSuccess) return -2;
-  return 0;
+  auto copy = [&](void* dst, const void* src, size_t bytes) {
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, s) == hipSuccess;
+  };
+  bool ok = !any_host || upload_step(*e);
+  for (const Input& in : inputs)
+    if (!in.host) ok = ok && copy(const_cast<void*>(in.dev), in.src, in.bytes);
+  if (!in_place)
+    ok = ok && copy(e->dec_key, key_cache, e->cache_bytes) && copy(e->dec_value, value_cache, e->cache_bytes);
+  ok = ok && launch_decoder_step(e->env(), sp, s) == hipSuccess &&
+       copy(logits, e->logits, (size_t)B * d.vocab * sizeof(float)) && copy(next_position, sp.next_pos, 8 * (size_t)B);
+  if (!in_place)
+    ok = ok && copy(key_cache, e->dec_key, e->cache_bytes) && copy(value_cache, e->dec_value, e->cache_bytes);
+  // also where something failed: the staging copy may still be read
+  return hipStreamSynchronize(s) == hipSuccess && ok ? 0 : -2;
 }
 
 extern "C" int32_t resident_epoch_prefill(void* engine, int32_t row, int32_t generation, const int64_t* prompt,
@@ -1340,46 +1407,29 @@ extern "C" int32_t resident_epoch_prefill(void* engine, int32_t row, int32_t gen
   std::lock_guard<std::mutex> lock(e->execute_mutex);
   hipStream_t s = e->stream;
   StepPtrs sp = e->step_io;
-  if (!copy_in(const_cast<int32_t*>(sp.table) + row * d.blocks_per_row, trow.data(), 4 * trow.size(), s)) return -2;
-  if (launch_clear_blocks(e->env(), e->key_cache, e->value_cache, sp.table + row * d.blocks_per_row,
-                          d.blocks_per_row, s) != hipSuccess)
-    return -2;
-  std::vector<int32_t> table((size_t)B * d.blocks_per_row, 0);
-  for (int j = 0; j < d.blocks_per_row; ++j) table[row * d.blocks_per_row + j] = trow[j];
-  std::vector<int64_t> tok(B, 0), pos(B, 0);
-  std::vector<int32_t> len(B, 0), slot(B, -1), act(B, 0);
+  std::memset(e->h_step, 0, e->step_in_bytes);
+  std::fill_n(staged(*e, sp.slot), B, -1);
+  std::copy(trow.begin(), trow.end(), staged(*e, sp.table) + row * d.blocks_per_row);
+  const bool cleared = upload_step(*e) && launch_clear_blocks(e->env(), e->key_cache, e->value_cache,
+                                                              sp.table + row * d.blocks_per_row, d.blocks_per_row,
+                                                              s) == hipSuccess;
+  // the staging copy changes below
+  if (hipStreamSynchronize(s) != hipSuccess || !cleared) return -2;
   sp.key_cache = e->key_cache;
   sp.value_cache = e->value_cache;
   sp.logits = e->logits;
   sp.done = nullptr;
   for (int p = 0; p + 1 < prompt_len; ++p) {
-    tok[row] = toks[p];
-    pos[row] = p;
-    len[row] = p + 1;
-    act[row] = 1;
-    const int lb = p / d.block_size;
-    slot[row] = trow[lb] * d.block_size + p % d.block_size;
-    // each step's inputs are staged synchronously: the host vectors change next iteration
-    bool ok = hipMemcpy(const_cast<int64_t*>(sp.token), tok.data(), 8 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(const_cast<int64_t*>(sp.pos), pos.data(), 8 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(const_cast<int32_t*>(sp.len), len.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(const_cast<int32_t*>(sp.slot), slot.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(const_cast<int32_t*>(sp.active), act.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(const_cast<int32_t*>(sp.table), table.data(), 4 * table.size(), hipMemcpyHostToDevice) ==
-                  hipSuccess;
-    if (!ok) return -2;
-    if (launch_decoder_step(e->env(), sp, s) != hipSuccess) return -2;
-    if (hipStreamSynchronize(s) != hipSuccess) return -2;
+    staged(*e, sp.token)[row] = toks[p];
+    staged(*e, sp.pos)[row] = p;
+    staged(*e, sp.len)[row] = p + 1;
+    staged(*e, sp.active)[row] = 1;
+    staged(*e, sp.slot)[row] = trow[p / d.block_size] * d.block_size + p % d.block_size;
+    const bool ok = upload_step(*e) && launch_decoder_step(e->env(), sp, s) == hipSuccess;
+    if (hipStreamSynchronize(s) != hipSuccess || !ok) return -2;
   }
-  const int32_t gen = generation, len_v = prompt_len, valid = 1;
-  const int64_t last_tok = toks[prompt_len - 1], last_pos = prompt_len - 1;
-  bool ok = hipMemcpy(e->st.res_gen + row, &gen, 4, hipMemcpyHostToDevice) == hipSuccess &&
-            hipMemcpy(e->st.res_token + row, &last_tok, 8, hipMemcpyHostToDevice) == hipSuccess &&
-            hipMemcpy(e->st.res_pos + row, &last_pos, 8, hipMemcpyHostToDevice) == hipSuccess &&
-            hipMemcpy(e->st.res_len + row, &len_v, 4, hipMemcpyHostToDevice) == hipSuccess &&
-            hipMemcpy(e->st.res_valid + row, &valid, 4, hipMemcpyHostToDevice) == hipSuccess &&
-            hipStreamSynchronize(s) == hipSuccess;
-  return ok ? 0 : -2;
+  const bool stored = store_rows(*e, {RowRecord{toks[prompt_len - 1], row, generation, prompt_len}});
+  return hipStreamSynchronize(s) == hipSuccess && stored ? 0 : -2;
 }
 
 namespace {
@@ -1431,7 +1481,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   const size_t o_mlp = take(M * I * T), o_rope = take((size_t)M * d.head_dim * sizeof(float));
   const size_t o_tok = take(8 * (size_t)M), o_pos = take(4 * (size_t)M), o_slot = take(4 * (size_t)M);
   const size_t o_tiles = take(sizeof(int4) * tiles.size()), o_blocks = take(4 * tables.size());
-  const size_t rows_bytes = off;
+  const size_t rows_bytes = off, tables_bytes = o_blocks + 4 * tables.size() - o_tok;
   // K ranges of the qkv, o and down GEMMs (bf16); each one's partial sums are
   // consumed before the next writes its own
   auto plan_of = [&](int N, int K) { return T == 2 && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
@@ -1452,13 +1502,19 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
     e.pf_bytes = off;
   }
   uint8_t* b = fixed != nullptr ? fixed : e.pf_mem;
-  const bool ok = (M == 0 || (hipMemcpy(b + o_tok, tok.data(), 8 * M, hipMemcpyHostToDevice) == hipSuccess &&
-                              hipMemcpy(b + o_pos, pos.data(), 4 * M, hipMemcpyHostToDevice) == hipSuccess &&
-                              hipMemcpy(b + o_slot, slot.data(), 4 * M, hipMemcpyHostToDevice) == hipSuccess &&
-                              hipMemcpy(b + o_tiles, tiles.data(), sizeof(int4) * tiles.size(),
-                                        hipMemcpyHostToDevice) == hipSuccess)) &&
-                  hipMemcpy(b + o_blocks, tables.data(), 4 * tables.size(), hipMemcpyHostToDevice) == hipSuccess;
-  if (!ok) return -2;
+  // The five tables lie back to back: one upload, and the rows' records are
+  // one more with a kernel (a blocking copy each, 25 for four rows, was 300 of
+  // the 430 us of four short prompts through two layers of the tiny model).
+  std::vector<uint8_t> up(tables_bytes);
+  auto stage = [&](size_t at, const auto& v) {
+    if (!v.empty()) std::memcpy(up.data() + (at - o_tok), v.data(), v.size() * sizeof(v[0]));
+  };
+  stage(o_tok, tok);
+  stage(o_pos, pos);
+  stage(o_slot, slot);
+  stage(o_tiles, tiles);
+  stage(o_blocks, tables);
+  if (hipMemcpyAsync(b + o_tok, up.data(), tables_bytes, hipMemcpyHostToDevice, s) != hipSuccess) return -2;
   const KernelEnv env = e.env();
   if (launch_clear_blocks(env, e.key_cache, e.value_cache, reinterpret_cast<const int32_t*>(b + o_blocks),
                           static_cast<int>(tables.size()), s) != hipSuccess)
@@ -1564,18 +1620,11 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
     }
     if (err != hipSuccess) return -2;
   }
-  if (hipStreamSynchronize(s) != hipSuccess) return -2;
-  for (int i = 0; i < nr; ++i) {
-    const int r = rows[i];
-    const int32_t len = static_cast<int32_t>(prompts[i].size()), valid = 1;
-    const int64_t last_tok = prompts[i].back(), last_pos = len - 1;
-    const bool stored = hipMemcpy(e.st.res_gen + r, &gens[i], 4, hipMemcpyHostToDevice) == hipSuccess &&
-                        hipMemcpy(e.st.res_token + r, &last_tok, 8, hipMemcpyHostToDevice) == hipSuccess &&
-                        hipMemcpy(e.st.res_pos + r, &last_pos, 8, hipMemcpyHostToDevice) == hipSuccess &&
-                        hipMemcpy(e.st.res_len + r, &len, 4, hipMemcpyHostToDevice) == hipSuccess &&
-                        hipMemcpy(e.st.res_valid + r, &valid, 4, hipMemcpyHostToDevice) == hipSuccess;
-    if (!stored) return -2;
-  }
+  std::vector<RowRecord> records;
+  for (int i = 0; i < nr; ++i)
+    records.push_back(RowRecord{prompts[i].back(), rows[i], gens[i], static_cast<int32_t>(prompts[i].size())});
+  const bool stored = store_rows(e, records);
+  if (hipStreamSynchronize(s) != hipSuccess || !stored) return -2;
   return 0;
 }
 
@@ -1678,16 +1727,18 @@ int32_t state_access(Engine* e, const char* name, void* buf, int64_t bytes, Acce
   } else if (n == "resident_rows") {
     const int B = d.batch;
     if (static_cast<size_t>(bytes) != 5 * 8 * (size_t)B) return -1;
-    std::vector<int32_t> gen(B), len(B), valid(B);
-    std::vector<int64_t> tok(B), pos(B), rows(5 * B);
+    // the five arrays lie back to back in the state buffer: one copy
+    uint8_t* base = reinterpret_cast<uint8_t*>(e->st.res_gen);
+    std::vector<uint8_t> img(reinterpret_cast<uint8_t*>(e->st.res_valid + B) - base);
+    auto at = [&](auto* dev) {
+      return reinterpret_cast<decltype(dev)>(img.data() + (reinterpret_cast<uint8_t*>(dev) - base));
+    };
+    int32_t *gen = at(e->st.res_gen), *len = at(e->st.res_len), *valid = at(e->st.res_valid);
+    int64_t *tok = at(e->st.res_token), *pos = at(e->st.res_pos);
+    std::vector<int64_t> rows(5 * B);
     if (hipStreamSynchronize(e->stream) != hipSuccess) return -2;
     if (mode == Access::kRead) {
-      bool ok = hipMemcpy(gen.data(), e->st.res_gen, 4 * B, hipMemcpyDeviceToHost) == hipSuccess &&
-                hipMemcpy(tok.data(), e->st.res_token, 8 * B, hipMemcpyDeviceToHost) == hipSuccess &&
-                hipMemcpy(pos.data(), e->st.res_pos, 8 * B, hipMemcpyDeviceToHost) == hipSuccess &&
-                hipMemcpy(len.data(), e->st.res_len, 4 * B, hipMemcpyDeviceToHost) == hipSuccess &&
-                hipMemcpy(valid.data(), e->st.res_valid, 4 * B, hipMemcpyDeviceToHost) == hipSuccess;
-      if (!ok) return -2;
+      if (hipMemcpy(img.data(), base, img.size(), hipMemcpyDeviceToHost) != hipSuccess) return -2;
       for (int r = 0; r < B; ++r) {
         rows[r] = gen[r];
         rows[B + r] = tok[r];
@@ -1705,12 +1756,7 @@ int32_t state_access(Engine* e, const char* name, void* buf, int64_t bytes, Acce
       len[r] = static_cast<int32_t>(rows[3 * B + r]);
       valid[r] = static_cast<int32_t>(rows[4 * B + r]);
     }
-    bool ok = hipMemcpy(e->st.res_gen, gen.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(e->st.res_token, tok.data(), 8 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(e->st.res_pos, pos.data(), 8 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(e->st.res_len, len.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(e->st.res_valid, valid.data(), 4 * B, hipMemcpyHostToDevice) == hipSuccess;
-    return ok ? 0 : -2;
+    return hipMemcpy(base, img.data(), img.size(), hipMemcpyHostToDevice) == hipSuccess ? 0 : -2;
   } else {
     auto it = e->weight_slots.find(n);
     if (it == e->weight_slots.end()) return -1;

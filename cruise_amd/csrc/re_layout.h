@@ -255,6 +255,13 @@ hipError_t launch_ctrl_init(const KernelEnv& env, const StatePtrs& st, int has_p
 hipError_t launch_clear_rows(const KernelEnv& env, const StatePtrs& st, void* key_cache,
                              void* value_cache, hipStream_t stream);
 hipError_t launch_ctrl_step(const KernelEnv& env, const StatePtrs& st, hipStream_t stream);
+// Resident record of a prefilled row: the next step's token at position
+// length - 1.
+struct RowRecord {
+  int64_t token;
+  int32_t row, generation, length;
+};
+hipError_t launch_store_rows(const StatePtrs& st, const RowRecord* rows, int n, hipStream_t stream);
 hipError_t launch_ctrl_finish(const KernelEnv& env, const StatePtrs& st, hipStream_t stream);
 // Import mode: Adler-32 of the imported blocks as they sit in the caches.
 hipError_t launch_import_checksum(const KernelEnv& env, const StatePtrs& st, const void* key_cache,

@@ -52,6 +52,8 @@ struct EmbedArgs {
   const int64_t* pos;
   const float* inv_freq;  // [d/2]
   float* rope;            // [B, d/2, 2] cos, sin (rounded to T)
+  const int32_t* active;
+  int64_t* next_pos;      // [B] where(active, pos + 1, pos), or null
   int B, H, V, half;
 };
 
@@ -61,6 +63,8 @@ __global__ void __launch_bounds__(256) k_embed(EmbedArgs a) {
   const int b = blockIdx.x, tid = threadIdx.x;
   long long t = a.token[b];
   if (t < 0 || t >= a.V) t = 0;  // the controller rejects such ids (CTRL:356); reads stay in bounds
+  // next_position (batched_decoder_step.py:409-411)
+  if (a.next_pos != nullptr && tid == 0) a.next_pos[b] = a.active[b] != 0 ? a.pos[b] + 1 : a.pos[b];
   for (int j = tid; j < a.half; j += blockDim.x) {
     const float ang = static_cast<float>(a.pos[b]) * a.inv_freq[j];
     a.rope[((size_t)b * a.half + j) * 2] = Elt<T>::r(cosf(ang));
@@ -808,6 +812,8 @@ static hipError_t decoder_step_t(const KernelEnv& env, const StepPtrs& st, hipSt
     e.pos = st.pos;
     e.inv_freq = sc.inv_freq;
     e.rope = sc.rope;
+    e.active = st.active;
+    e.next_pos = st.next_pos;
     e.B = B;
     e.H = d.hidden;
     e.V = d.vocab;
