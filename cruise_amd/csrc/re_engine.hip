@@ -1600,6 +1600,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       at.heads = d.heads;
       at.kv_heads = d.kv_heads;
       at.head_dim = d.head_dim;
+      at.max_keys = *std::max_element(pos.begin(), pos.end()) + 1;
       run(launch_prefill_attention(at, d, static_cast<int>(tiles.size()), s));
       gemm(o_attn, d.q_dim(), lo.o_w, SIZE_MAX, o_hidden, d.hidden, d.hidden, d.q_dim(), kGemmResidual, o_plan);
       norm(lo.post_norm, o_plan);

@@ -308,6 +308,7 @@ struct PrefillAttn {           // causal attention within each row's prompt
   const int32_t* pos;          // [M]
   const int4* tiles;           // MFMA path: {first query token, row's first token, queries, first position}
   int M, ld, heads, kv_heads, head_dim;
+  int max_keys;                // longest prompt of the pass (prefilled tokens)
 };
 // Store: out = T(acc + bias); Residual: out = T(out + T(acc)); SwiGlu: W holds
 // the gate rows and W2 the up rows, and out[m, n] =

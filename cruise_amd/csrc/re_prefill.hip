@@ -23,6 +23,7 @@
 //              (token, head).
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "re_device.h"
 #include "re_layout.h"
@@ -773,7 +774,15 @@ constexpr int kAvld = kAd + 16;  // V tile row stride: 4 key rows of a transposi
 //     row-major V tile by transposing LDS reads.  The two key halves'
 //     partial O are added at the end.
 // LDS: one K tile and one V tile (35 KB), independent of the prompt length.
-constexpr int kFlashLds = kAk * kAkld * 2 + kAk * kAvld * 2;
+//
+// NT > 0, for prompts of up to NT key tiles: pass 1 keeps its scores for pass
+// 2, packed (they are bf16 values: 8 registers a tile and lane), in loops
+// unrolled so that the registers have fixed names.  Pass 2 then reads value
+// tiles alone, one barrier each, from two LDS buffers (the second lies over
+// the key tile); the first is on its way during pass 1's last tile.  What
+// bounds short prompts is the chain of waits, not the work: FLASH_FIG
+constexpr int kFlashLds = 2 * kAk * kAvld * 2;
+static_assert(kAk * kAkld * 2 <= kAk * kAvld * 2, "the key tile fits the first value buffer");
 
 // Workgroup order: the (KV head, query tile) pairs P = g * ntiles + t are cut
 // into chunks of kFlashChunk consecutive tiles (a 1000-token prompt's tiles
@@ -784,16 +793,25 @@ constexpr int kFlashLds = kAk * kAkld * 2 + kAk * kAvld * 2;
 // heads, instead of from the memory-side cache once per head.
 constexpr int kFlashChunk = 16;
 
+constexpr int kFlashKept = 16;  // key tiles whose scores fit the registers (242 of 256)
+
 int flash_grid(int ntiles, int heads, int kv_heads) {
   const int chunks = (ntiles * kv_heads + kFlashChunk - 1) / kFlashChunk;
   return (chunks + 7) / 8 * 8 * kFlashChunk * (heads / kv_heads);
 }
 
+// f(0), f(1), ... with the index a constant.
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_index(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int NT>
 __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int ntiles) {
   __shared__ __align__(16) unsigned char smem[kFlashLds];
   __shared__ float stat[2][2][32][2];  // [query half][key half][query][max, sum]
   bf16_t* Ks = reinterpret_cast<bf16_t*>(smem);  // [64 keys][136]
-  bf16_t* Vs = Ks + kAk * kAkld;                  // [64 keys][144]
+  bf16_t* Vs = Ks + kAk * kAvld;                  // [64 keys][144]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int tix, h;
   {
@@ -839,12 +857,12 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
       kpre[i] = *reinterpret_cast<const re_u32x4*>(qkv + (size_t)tok * a.ld + koff + (v & 15) * 8);
     }
   };
-  auto load_v = [&](int kt) {
+  auto load_v = [&](int kt, re_u32x4 (&dst)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int v = tid + 256 * i;
       const int tok = r0 + min(min(kt, nkt - 1) * kAk + (v & 63), nkeys - 1);
-      vpre[i] = *reinterpret_cast<const re_u32x4*>(qkv + (size_t)tok * a.ld + voff + (v >> 6) * 8);
+      dst[i] = *reinterpret_cast<const re_u32x4*>(qkv + (size_t)tok * a.ld + voff + (v >> 6) * 8);
     }
   };
   auto store_k = [&]() {
@@ -854,18 +872,15 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
       *reinterpret_cast<re_u32x4*>(&Ks[(v >> 4) * kAkld + (v & 15) * 8]) = kpre[i];
     }
   };
-  auto store_v = [&]() {
+  auto store_v = [&](bf16_t* V, const re_u32x4 (&src)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int v = tid + 256 * i, key = v & 63, c = (v >> 6) * 8;
-      *reinterpret_cast<re_u32x4*>(&Vs[key * kAvld + c]) = vpre[i];
+      *reinterpret_cast<re_u32x4*>(&V[key * kAvld + c]) = src[i];
     }
   };
-  // Scores of key tile kt for this lane's query: s[v] is key
-  // kt * 64 + sn * 32 + 8 (v / 4) + 4 hi + v % 4.  MASKED: the tile reaches
-  // past some query's causal limit (the tiles before nfull end at or before
-  // the first query's position, so every query sees all of their keys).
-  auto scores = [&](int kt, float (&sc)[16], auto masked) {
+  // This wave's K Q^T of the key tile in LDS.
+  auto key_products = [&]() {
     f32x16_t acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.f;
@@ -874,6 +889,14 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
       const bf16x8_t kf = lds_frag(&Ks[(sn * 32 + (lane & 31)) * kAkld + ks * 16 + hi * 8]);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], acc, 0, 0, 0);
     }
+    return acc;
+  };
+  // Scores of key tile kt for this lane's query: s[v] is key
+  // kt * 64 + sn * 32 + 8 (v / 4) + 4 hi + v % 4.  MASKED: the tile reaches
+  // past some query's causal limit (the tiles before nfull end at or before
+  // the first query's position, so every query sees all of their keys).
+  auto scores = [&](int kt, float (&sc)[16], auto masked) {
+    const f32x16_t acc = key_products();
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const float x = round_bf16(div_sqrt128_bf16(round_bf16(acc[v])));
@@ -890,13 +913,8 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
   // Pass 1: row max and sum.  A masked score adds exp2(-inf) = 0; while all
   // of a lane's scores so far are masked (m = -inf) its sum stays 0.
   float m = -INFINITY, l = 0.f;
-  auto pass1 = [&](int kt, auto masked) {
+  auto accumulate = [&](const float (&sc)[16]) {
 #pragma clang fp contract(off)  // the rescaled sum is a product, then a sum
-    store_k();
-    load_k(kt + 1);
-    lds_barrier();
-    float sc[16];
-    scores(kt, sc, masked);
     float tmax = sc[0];
 #pragma unroll
     for (int v = 1; v < 16; ++v) tmax = fmaxf(tmax, sc[v]);
@@ -907,10 +925,56 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
     for (int v = 0; v < 16; ++v) add += __builtin_amdgcn_exp2f(fmaf(sc[v], kLog2e, -bn));
     l = l * __builtin_amdgcn_exp2f(fmaf(m, kLog2e, -bn)) + add;
     m = mn;
+  };
+  auto pass1 = [&](int kt, auto masked) {
+    store_k();
+    load_k(kt + 1);
+    lds_barrier();
+    float sc[16];
+    scores(kt, sc, masked);
+    accumulate(sc);
     lds_barrier();
   };
+  uint32_t kept[NT > 0 ? NT : 1][8];  // scores 2 i, 2 i + 1 of each key tile
+  auto kept_scores = [&](const uint32_t (&k)[8], float (&sc)[16]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      sc[2 * i] = __uint_as_float(k[i] << 16);
+      sc[2 * i + 1] = __uint_as_float(k[i] & 0xffff0000u);
+    }
+  };
   load_k(0);
-  {
+  if constexpr (NT > 0) {
+    auto tile = [&](auto index) __attribute__((always_inline)) {
+      constexpr int kt = decltype(index)::value;
+      if (kt >= nkt) return;
+      store_k();
+      if (kt + 1 < nkt)
+        load_k(kt + 1);
+      else
+        load_v(0, kpre);
+      lds_barrier();
+      const f32x16_t acc = key_products();
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        kept[kt][i] = f2_to_bf16x2_raw(div_sqrt128_bf16(round_bf16(acc[2 * i])), div_sqrt128_bf16(round_bf16(acc[2 * i + 1])));
+      float sc[16];
+      kept_scores(kept[kt], sc);
+      if (kt >= nfull) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int j = kt * kAk + sn * 32 + 8 * (i >> 1) + 4 * hi + 2 * (i & 1);
+          if (j > qlim) kept[kt][i] = (kept[kt][i] & 0xffff0000u) | 0xff80u;
+          if (j + 1 > qlim) kept[kt][i] = (kept[kt][i] & 0xffffu) | 0xff800000u;
+        }
+        kept_scores(kept[kt], sc);
+      }
+      accumulate(sc);
+      if (kt + 1 < nkt) lds_barrier();
+    };
+    for_each_index(tile, std::make_integer_sequence<int, NT>{});
+    store_v(Vs, kpre);  // behind the key tile; complete at the statistics' barrier
+  } else {
     int kt = 0;
     for (; kt < nfull; ++kt) pass1(kt, std::false_type{});
     for (; kt < nkt; ++kt) pass1(kt, std::true_type{});
@@ -950,14 +1014,7 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
     for (int v = 0; v < 16; ++v) o[t][v] = 0.f;
   // M is finite (key 0 is visible to every query), so a masked score's
   // probability is exp2(-inf) = 0.
-  auto pass2 = [&](int kt, auto masked) {
-    store_k();
-    store_v();
-    load_k(kt + 1);
-    load_v(kt + 1);
-    lds_barrier();
-    float sc[16];
-    scores(kt, sc, masked);
+  auto add_values = [&](const float (&sc)[16], const bf16_t* V) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       float pv[8];
@@ -975,7 +1032,7 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
       const int gi = lane & 15, q4 = (gi & 3) * 4, rr = gi >> 2, d16 = ((lane >> 4) & 1) * 16;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const bf16_t* vr = &Vs[(kb + rr) * kAvld + t * 32 + d16 + q4];
+        const bf16_t* vr = &V[(kb + rr) * kAvld + t * 32 + d16 + q4];
         const lds_v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)vr);
         const lds_v4i16 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(vr + 8 * kAvld));
         const uint2 l2 = __builtin_bit_cast(uint2, lo), u2 = __builtin_bit_cast(uint2, up);
@@ -983,11 +1040,33 @@ __global__ void __launch_bounds__(256, 2) k_pf_attn_flash(PrefillAttn a, int nti
         o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8_t, bw), o[t], 0, 0, 0);
       }
     }
+  };
+  auto pass2 = [&](int kt, auto masked) {
+    store_k();
+    store_v(Vs, vpre);
+    load_k(kt + 1);
+    load_v(kt + 1, vpre);
+    lds_barrier();
+    float sc[16];
+    scores(kt, sc, masked);
+    add_values(sc, Vs);
     lds_barrier();
   };
-  load_k(0);
-  load_v(0);
-  {
+  if constexpr (NT > 0) {
+    auto tile = [&](auto index) __attribute__((always_inline)) {
+      constexpr int kt = decltype(index)::value;
+      if (kt >= nkt) return;
+      if (kt + 1 < nkt) load_v(kt + 1, kpre);
+      float sc[16];
+      kept_scores(kept[kt], sc);
+      add_values(sc, kt % 2 == 0 ? Vs : Ks);
+      if (kt + 1 < nkt) store_v(kt % 2 == 0 ? Ks : Vs, kpre);
+      lds_barrier();
+    };
+    for_each_index(tile, std::make_integer_sequence<int, NT>{});
+  } else {
+    load_k(0);
+    load_v(0, vpre);
     int kt = 0;
     for (; kt < nfull; ++kt) pass2(kt, std::false_type{});
     for (; kt < nkt; ++kt) pass2(kt, std::true_type{});
@@ -1188,7 +1267,15 @@ hipError_t launch_prefill_attention(const PrefillAttn& a, const Dims& d, int nti
   if (prefill_attention_mfma(d)) {
     if (ntiles <= 0) return hipErrorInvalidValue;
     if (d.heads % d.kv_heads != 0) return hipErrorInvalidValue;
-    k_pf_attn_flash<<<flash_grid(ntiles, d.heads, d.kv_heads), 256, 0, stream>>>(a, ntiles);
+    const int grid = flash_grid(ntiles, d.heads, d.kv_heads), key_tiles = (a.max_keys + kAk - 1) / kAk;
+    if (key_tiles <= 1)
+      k_pf_attn_flash<1><<<grid, 256, 0, stream>>>(a, ntiles);
+    else if (key_tiles <= 4)
+      k_pf_attn_flash<4><<<grid, 256, 0, stream>>>(a, ntiles);
+    else if (key_tiles <= kFlashKept)
+      k_pf_attn_flash<kFlashKept><<<grid, 256, 0, stream>>>(a, ntiles);
+    else
+      k_pf_attn_flash<0><<<grid, 256, 0, stream>>>(a, ntiles);
   } else {
     if (256 % d.head_dim != 0 || d.head_dim % 8 != 0) return hipErrorInvalidValue;
     const size_t bytes = (size_t)d.capacity * sizeof(float);
