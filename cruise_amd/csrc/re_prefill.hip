@@ -6,7 +6,7 @@
 //   rmsnorm    one workgroup per token
 //   GEMM       C[M,N] = A[M,K] W[N,K]^T, both operands K-contiguous.
 //              bf16: MFMA v_mfma_f32_16x16x32_bf16, workgroup tiles of 256
-//              columns by 64 to 256 rows, K in steps of 64 through LDS
+//              (or 192) columns by 64 to 256 rows, K in steps of 64 through LDS
 //              stages filled by direct global -> LDS loads, fp32
 //              accumulation; epilogues "T(acc + bias)", the residual
 //              "T(h + T(acc))", and gate/up with SwiGLU in one GEMM (the
@@ -274,15 +274,16 @@ __global__ void __launch_bounds__(PART ? 512 : 256) k_pf_qkv_post(PrefillQkv a) 
 // Requirements (checked by launch_gemm): K % 64 == 0, N % 8 == 0, lda, ldw
 // and ldo multiples of 8 elements, 16-byte aligned operands.
 constexpr int kGn = 256, kGk = 64;
+constexpr int kGnNarrow = 192;
 constexpr int kGrowBytes = kGk * 2;                   // one K step of one row
 constexpr int kGwaves = 8, kGthreads = kGwaves * 64;
-constexpr int kGoutLd = kGn + 8;                      // epilogue row stride (elements)
 constexpr int kGgroupM = 4;
 constexpr int gemm_tile_m(int mj) { return 64 * mj; }
-constexpr int gemm_stage_bytes(int mj) { return (kGn + gemm_tile_m(mj)) * kGrowBytes; }
+constexpr int gemm_stage_bytes(int mj, int gn) { return (gn + gemm_tile_m(mj)) * kGrowBytes; }
 constexpr int gemm_stages(int mj) { return mj <= 2 ? 3 : 2; }
-constexpr int gemm_lds_bytes(int mj, int st) {
-  return std::max(gemm_tile_m(mj) * kGoutLd * 2, st * gemm_stage_bytes(mj));
+constexpr int gemm_out_ld(int gn) { return gn + 8; }  // epilogue row stride (elements)
+constexpr int gemm_lds_bytes(int mj, int st, int gn) {
+  return std::max(gemm_tile_m(mj) * gemm_out_ld(gn) * 2, st * gemm_stage_bytes(mj, gn));
 }
 
 typedef const __attribute__((address_space(1))) void* gemm_gptr;
@@ -337,20 +338,20 @@ constexpr int gemm_reads_by(int frags, int prods, int p) {
   return n < frags ? n : frags;
 }
 
-template <int EPI, int MJ, int ST>
+template <int EPI, int MJ, int ST, int GN>
 __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, int nN, int nS) {
   extern __shared__ __align__(16) unsigned char gsm[];
-  constexpr int kTm = gemm_tile_m(MJ), kStage = gemm_stage_bytes(MJ);
-  constexpr int kInsts = 4 + MJ;  // 1 KB loads (8 rows) of each wave and stage
+  constexpr int kTm = gemm_tile_m(MJ), kStage = gemm_stage_bytes(MJ, GN), kOutLd = gemm_out_ld(GN);
+  constexpr int kWInsts = GN / 64, kInsts = kWInsts + MJ;  // 1 KB loads (8 rows) of each wave and stage
   // wave-uniform, so the load base lives in SGPRs (32-bit per-lane offsets)
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
   int mt, nt, ks;
   gemm_tile_of(blockIdx.x, nM, nN, nS, mt, nt, ks);
-  // The SwiGLU tile covers 128 output columns: W tile rows 0..127 are their
-  // gate rows, rows 128..255 their up rows.
+  // The SwiGLU tile covers GN / 2 output columns: the first half of the W tile
+  // rows are their gate rows, the second half their up rows.
   constexpr bool kPart = EPI == kGemmPart;
   constexpr bool kSwiGlu = EPI == kGemmSwiGlu;
-  constexpr int kTileN = kSwiGlu ? kGn / 2 : kGn;
+  constexpr int kTileN = kSwiGlu ? GN / 2 : GN;
   const int m0 = mt * kTm, n0 = nt * kTileN;
   // K steps of this workgroup: range ks of nS nearly equal ones
   const int steps = a.K / kGk;
@@ -360,6 +361,7 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   // 0..255.  Smaller ones: every wave 32 W rows (4 loads) and 8 MJ A rows.
   // Rows past M or N read a valid row (clamped) whose results are never stored.
   constexpr bool kSplitLoads = MJ == 4;
+  static_assert(!kSplitLoads || GN == kGn, "256-row tiles are 256 wide");
   const char* wbase;
   const char* abase = static_cast<const char*>(a.A) + (size_t)m0 * a.lda * 2 + (size_t)k_begin * kGrowBytes;
   uint32_t goff[kInsts];
@@ -381,16 +383,16 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
     }
     lrow[0] = lrow[1] = row0;
   } else {
-    lrow[0] = wave * 32;
-    lrow[1] = kGn + wave * 8 * MJ;
+    lrow[0] = wave * (GN / 8);
+    lrow[1] = GN + wave * 8 * MJ;
     const void* wsrc = kSwiGlu && lrow[0] >= kTileN ? a.W2 : a.W;
     wbase = static_cast<const char*>(wsrc) + (size_t)n0 * a.ldw * 2 + (size_t)k_begin * kGrowBytes;
 #pragma unroll
     for (int i = 0; i < kInsts; ++i) {
-      const int row = (i < 4 ? lrow[0] + i * 8 : lrow[1] + (i - 4) * 8) + (lane >> 3);
+      const int row = (i < kWInsts ? lrow[0] + i * 8 : lrow[1] + (i - kWInsts) * 8) + (lane >> 3);
       const int chunk = (lane & 7) ^ gemm_swz(row);
-      goff[i] = i < 4 ? static_cast<uint32_t>(min(row % kTileN, a.N - n0 - 1) * a.ldw * 2 + chunk * 16)
-                      : static_cast<uint32_t>(min(row - kGn, a.M - m0 - 1) * a.lda * 2 + chunk * 16);
+      goff[i] = i < kWInsts ? static_cast<uint32_t>(min(row % kTileN, a.N - n0 - 1) * a.ldw * 2 + chunk * 16)
+                      : static_cast<uint32_t>(min(row - GN, a.M - m0 - 1) * a.lda * 2 + chunk * 16);
     }
   }
   auto issue = [&](int kt, int buf) {
@@ -403,16 +405,16 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
                                          (gemm_lptr)(l + lrow[0] * kGrowBytes + i * 1024), 16, 0, 0);
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < kWInsts; ++i)
         __builtin_amdgcn_global_load_lds((gemm_gptr)(wbase + kb + goff[i]),
                                          (gemm_lptr)(l + lrow[0] * kGrowBytes + i * 1024), 16, 0, 0);
 #pragma unroll
-      for (int i = 4; i < kInsts; ++i)
+      for (int i = kWInsts; i < kInsts; ++i)
         __builtin_amdgcn_global_load_lds((gemm_gptr)(abase + kb + goff[i]),
-                                         (gemm_lptr)(l + lrow[1] * kGrowBytes + (i - 4) * 1024), 16, 0, 0);
+                                         (gemm_lptr)(l + lrow[1] * kGrowBytes + (i - kWInsts) * 1024), 16, 0, 0);
     }
   };
-  constexpr int kWn = gemm_waves_n(MJ), NI = 16 / kWn, MI = 4 * MJ / (kGwaves / kWn);
+  constexpr int kWn = gemm_waves_n(MJ), NI = GN / 16 / kWn, MI = 4 * MJ / (kGwaves / kWn);
   const int wn = wave % kWn, wm = wave / kWn;
   f32x4_t acc[NI][MI];
 #pragma unroll
@@ -433,7 +435,7 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   constexpr int kFrags = NI + MI, kProds = NI * MI;
   bf16x8_t f[2][kFrags];
   auto read_frag = [&](int set, int idx, int st, int ks2) {
-    f[set][idx] = idx < NI ? frag(st, (wn * NI + idx) * 16, ks2) : frag(st, kGn + (wm * MI + idx - NI) * 16, ks2);
+    f[set][idx] = idx < NI ? frag(st, (wn * NI + idx) * 16, ks2) : frag(st, GN + (wm * MI + idx - NI) * 16, ks2);
   };
   auto read_set = [&](int set, int st, int ks2) {
 #pragma unroll
@@ -531,7 +533,7 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
         y[2] += __uint_as_float(b.y << 16);
         y[3] += __uint_as_float(b.y & 0xffff0000u);
       }
-      *reinterpret_cast<uint2*>(T + ml * kGoutLd + nl) =
+      *reinterpret_cast<uint2*>(T + ml * kOutLd + nl) =
           make_uint2(f_to_bf16(y[0]) | ((uint32_t)f_to_bf16(y[1]) << 16),
                      f_to_bf16(y[2]) | ((uint32_t)f_to_bf16(y[3]) << 16));
     }
@@ -546,8 +548,8 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
       const int r = idx / (kTileN / 8), c = idx % (kTileN / 8);
       const int m = m0 + r, n = n0 + c * 8;
       if (m >= a.M || n >= a.N) continue;
-      const Vec8<bf16_t> gv = Vec8<bf16_t>::load_cached(T + r * kGoutLd + c * 8);
-      const Vec8<bf16_t> uv = Vec8<bf16_t>::load_cached(T + r * kGoutLd + kTileN + c * 8);
+      const Vec8<bf16_t> gv = Vec8<bf16_t>::load_cached(T + r * kOutLd + c * 8);
+      const Vec8<bf16_t> uv = Vec8<bf16_t>::load_cached(T + r * kOutLd + kTileN + c * 8);
       float y[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -560,11 +562,11 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
     return;
   }
 #pragma unroll 4
-  for (int idx = tid; idx < kTm * kGn / 8; idx += kGthreads) {
-    const int r = idx / (kGn / 8), c = idx % (kGn / 8);
+  for (int idx = tid; idx < kTm * GN / 8; idx += kGthreads) {
+    const int r = idx / (GN / 8), c = idx % (GN / 8);
     const int m = m0 + r, n = n0 + c * 8;
     if (m >= a.M || n >= a.N) continue;
-    re_u32x4 t = *reinterpret_cast<const re_u32x4*>(T + r * kGoutLd + c * 8);
+    re_u32x4 t = *reinterpret_cast<const re_u32x4*>(T + r * kOutLd + c * 8);
     re_u32x4* p = reinterpret_cast<re_u32x4*>(out + (size_t)m * a.ldo + n);
     if constexpr (EPI == kGemmResidual) {
       const re_u32x4 h = *p;
@@ -1137,19 +1139,33 @@ hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStre
   return hipGetLastError();
 }
 
-template <int EPI, int MJ>
+template <int EPI, int MJ, int GN = kGn>
 static hipError_t gemm_launch(const GemmArgs& a, int splits, hipStream_t stream) {
-  constexpr int ST = gemm_stages(MJ), kLds = gemm_lds_bytes(MJ, ST);
-  constexpr int kTileN = EPI == kGemmSwiGlu ? kGn / 2 : kGn;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_bf16<EPI, MJ, ST>),
+  constexpr int ST = gemm_stages(MJ), kLds = gemm_lds_bytes(MJ, ST, GN);
+  constexpr int kTileN = EPI == kGemmSwiGlu ? GN / 2 : GN;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_bf16<EPI, MJ, ST, GN>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   if (attr != hipSuccess) return attr;
   const int nM = (a.M + gemm_tile_m(MJ) - 1) / gemm_tile_m(MJ), nN = (a.N + kTileN - 1) / kTileN;
-  k_gemm_bf16<EPI, MJ, ST><<<nM * nN * splits, kGthreads, kLds, stream>>>(a, nM, nN, splits);
+  k_gemm_bf16<EPI, MJ, ST, GN><<<nM * nN * splits, kGthreads, kLds, stream>>>(a, nM, nN, splits);
   return hipGetLastError();
 }
+// Gate/up of up to 192 tokens: its tiles of 128 columns are one row of them,
+// fewer than the CUs (148 of 256 at the 7B shape), and a CU takes a stage's W
+// rows no faster for the idle ones.  Tiles of 96 columns where they fit the CUs
+// in one round too (198): 10 tokens 54.3 -> 49.0 us, 64 tokens 61.8 -> 53.8, 65
+// 66.4 -> 56.6, 128 72.4 -> 64.7, 160 99.3 -> 91.4.  256-row tiles gain nothing
+// (220 tokens 100.5 and 99.7), and stay.
 template <int EPI>
 static hipError_t gemm_launch_mj(const GemmArgs& a, const GemmPlan& p, hipStream_t stream) {
+  if constexpr (EPI == kGemmSwiGlu) {
+    constexpr int kCols = kGnNarrow / 2, kCus = 256;
+    if (a.M <= gemm_tile_m(p.mj) && (a.N + kCols - 1) / kCols <= kCus) {
+      if (p.mj == 1) return gemm_launch<EPI, 1, kGnNarrow>(a, 1, stream);
+      if (p.mj == 2) return gemm_launch<EPI, 2, kGnNarrow>(a, 1, stream);
+      if (p.mj == 3) return gemm_launch<EPI, 3, kGnNarrow>(a, 1, stream);
+    }
+  }
   switch (p.mj) {
     case 1: return gemm_launch<EPI, 1>(a, p.splits, stream);
     case 2: return gemm_launch<EPI, 2>(a, p.splits, stream);
