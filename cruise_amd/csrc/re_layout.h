@@ -231,7 +231,7 @@ int timed_op_index(const KernelEnv& env, int layer);
 void plan_grids(LaunchPlan& p, const Dims& d, int cus);
 // Decode projections on the matrix cores at 64 batch rows (re_mfma.hip):
 // the RMSNorm (where the projection has one) and the projection of one op.
-enum class MfmaOp { kQkv, kO, kGateUp, kDown, kLmHead };
+enum class MfmaOp { kEmbed, kQkv, kO, kGateUp, kDown, kLmHead };
 bool mfma_step_supported(const Dims& d);
 int mfma_lm_partials(const Dims& d);
 bool mfma_lm_cu_fits(const Dims& d, int cus);

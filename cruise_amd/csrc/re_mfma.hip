@@ -28,7 +28,8 @@
 // column l % 16.
 //
 // The RMSNorm before qkv, gate/up and the LM head runs as its own kernel
-// (one workgroup per row) into a normalized copy of the rows.
+// (one workgroup per row) into a normalized copy of the rows; the first one
+// takes the step's embedding rows with it.
 #include <type_traits>
 
 #include "re_device.h"
@@ -527,59 +528,96 @@ __global__ void __launch_bounds__(256) k_mf_qkv_finish(MfArgs a) {
 // first: h = T(h + T(p_0 + p_1 + ... )) over its fp32 partials in range order
 // (batched_decoder_step.py:380-386, 399-403), written back to the residual
 // stream, then normalized.
-template <int PARTS>
-__global__ void __launch_bounds__(256) k_mf_norm(const int32_t* done, bf16_t* h, const bf16_t* w, bf16_t* y,
-                                               int H, float eps, const float* part, int B) {
-  __shared__ float red[4];
-  if (done != nullptr && __builtin_nontemporal_load(done) != 0) return;
-  const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
-  bf16_t* hr = h + (size_t)m * H;
-  constexpr int kMaxChunks = 4;  // H <= 4 * 256 * 8
-  Vec8<bf16_t> hv[kMaxChunks];
+//
+// EMBED: the step's first launch; the row is the token's embedding, written to
+// the residual stream, with the step's RoPE table and next_position as k_embed
+// (re_step.hip) leaves them.
+//
+// One workgroup per row, a thread per 8 elements: everything a row needs is
+// requested at once, so the launch is one round trip to memory and the
+// reduction.  16 rows: 5.3 -> 5.1 us with partials; the embedding and the first
+// norm were two launches of 4.8 and 4.7 us and are one of 4.7.
+struct MfNormArgs {
+  const int32_t* done;
+  bf16_t* h;
+  const bf16_t* w;
+  bf16_t* y;
+  float eps;
+  const float* part;  // [PARTS][B][H]
+  int B;
+  // EMBED
+  const int64_t* token;
+  const int64_t* pos;
+  const bf16_t* embedding;
+  const float* inv_freq;  // [half]
+  float* rope;            // [B, half, 2]
+  const int32_t* active;
+  int64_t* next_pos;      // or null
+  int V, half;
+};
+
+constexpr int kNormThreads = kMfHidden / 8;
+static_assert(kNormThreads % 64 == 0, "whole waves");
+
+template <int PARTS, bool EMBED>
+__global__ void __launch_bounds__(kNormThreads) k_mf_norm(MfNormArgs a) {
+  constexpr int H = kMfHidden, kWaves = kNormThreads / 64;
+  __shared__ float red[kWaves];
+  const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid), c = tid * 8;
+  const int32_t stop = a.done != nullptr ? request_flag(a.done) : 0;
+  bf16_t* hr = a.h + (size_t)m * H + c;
+  const Vec8<bf16_t> wv = Vec8<bf16_t>::load_cached(a.w + c);
+  Vec8<bf16_t> hv;
+  if constexpr (EMBED) {
+    long long t = a.token[m];
+    if (t < 0 || t >= a.V) t = 0;  // the controller rejects such ids (CTRL:356); reads stay in bounds
+    hv = Vec8<bf16_t>::load_cached(a.embedding + (size_t)t * H + c);
+  } else {
+    hv = Vec8<bf16_t>::load_cached(hr);
+  }
+  re_f32x4 pv[PARTS > 0 ? PARTS : 1][2];
+#pragma unroll
+  for (int r = 0; r < PARTS; ++r) {
+    const float* p = a.part + ((size_t)r * a.B + m) * H + c;
+    pv[r][0] = *reinterpret_cast<const re_f32x4*>(p);
+    pv[r][1] = *reinterpret_cast<const re_f32x4*>(p + 4);
+  }
+  if (flag_set(stop)) return;
+  if constexpr (EMBED) {
+    const int64_t pos = a.pos[m];
+    for (int j = tid; j < a.half; j += kNormThreads) {
+      const float ang = static_cast<float>(pos) * a.inv_freq[j];
+      a.rope[((size_t)m * a.half + j) * 2] = round_bf16(cosf(ang));
+      a.rope[((size_t)m * a.half + j) * 2 + 1] = round_bf16(sinf(ang));
+    }
+    if (a.next_pos != nullptr && tid == 0) a.next_pos[m] = a.active[m] != 0 ? pos + 1 : pos;
+  }
+  if constexpr (PARTS > 0) {
+    float nh[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float sum = pv[0][e >> 2][e & 3];
+#pragma unroll
+      for (int r = 1; r < PARTS; ++r) sum += pv[r][e >> 2][e & 3];
+      nh[e] = bf16_to_f(f_to_bf16(hv.get(e) + round_bf16(sum)));
+    }
+    hv = Vec8<bf16_t>::from_floats(nh);
+  }
+  if constexpr (PARTS > 0 || EMBED) *reinterpret_cast<Vec8<bf16_t>*>(hr) = hv;
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < kMaxChunks; ++i) {
-    const int ch = tid + 256 * i;
-    hv[i] = ch * 8 < H ? Vec8<bf16_t>::load_cached(hr + ch * 8) : Vec8<bf16_t>{};
-    if (PARTS > 0 && ch * 8 < H) {
-      // all PARTS partials requested at once, then added in order
-      re_f32x4 pv[PARTS > 0 ? PARTS : 1][2];
-      const float* p0 = part + (size_t)m * H + ch * 8;
-#pragma unroll
-      for (int r = 0; r < PARTS; ++r) {
-        pv[r][0] = *reinterpret_cast<const re_f32x4*>(p0 + (size_t)r * B * H);
-        pv[r][1] = *reinterpret_cast<const re_f32x4*>(p0 + (size_t)r * B * H + 4);
-      }
-      float sum[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) sum[e] = pv[0][e >> 2][e & 3];
-#pragma unroll
-      for (int r = 1; r < PARTS; ++r)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sum[e] += pv[r][e >> 2][e & 3];
-      float nh[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) nh[e] = bf16_to_f(f_to_bf16(hv[i].get(e) + round_bf16(sum[e])));
-      hv[i] = Vec8<bf16_t>::from_floats(nh);
-      *reinterpret_cast<Vec8<bf16_t>*>(hr + ch * 8) = hv[i];
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s = fmaf(hv[i].get(e), hv[i].get(e), s);
-  }
+  for (int e = 0; e < 8; ++e) s = fmaf(hv.get(e), hv.get(e), s);
   s = wave_sum(s);
   if (lane == 0) red[wave] = s;
   __syncthreads();
-  const float rs = rsqrtf((red[0] + red[1] + red[2] + red[3]) / static_cast<float>(H) + eps);
+  float total = red[0];
 #pragma unroll
-  for (int i = 0; i < kMaxChunks; ++i) {
-    const int ch = tid + 256 * i;
-    if (ch * 8 >= H) continue;
-    const Vec8<bf16_t> wv = Vec8<bf16_t>::load_cached(w + ch * 8);
-    float out[8];
+  for (int i = 1; i < kWaves; ++i) total += red[i];
+  const float rs = rsqrtf(total / static_cast<float>(H) + a.eps);
+  float out[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = round_bf16(round_bf16(hv[i].get(e) * rs) * wv.get(e));
-    *reinterpret_cast<Vec8<bf16_t>*>(y + xpack_index(m, ch * 8, H)) = Vec8<bf16_t>::from_floats(out);
-  }
+  for (int e = 0; e < 8; ++e) out[e] = round_bf16(round_bf16(hv.get(e) * rs) * wv.get(e));
+  *reinterpret_cast<Vec8<bf16_t>*>(a.y + xpack_index(m, c, H)) = Vec8<bf16_t>::from_floats(out);
 }
 
 // The packed copy of one [rows, K] matrix: 16-byte unit u = (strip * K/32 +
@@ -716,17 +754,21 @@ hipError_t prepare_mfma(const Dims& d) {
   return e;
 }
 
-// The RMSNorm launch; with pending (o or down split) partials it adds them first.
-static void mf_norm(const KernelEnv& env, const StepPtrs& st, size_t w_off, bool pending, hipStream_t stream) {
-  const Dims& d = env.dims;
-  const Scratch& sc = env.scratch;
-  bf16_t* h = static_cast<bf16_t*>(sc.hidden);
-  const bf16_t* w = reinterpret_cast<const bf16_t*>(env.weights + w_off);
-  bf16_t* y = static_cast<bf16_t*>(sc.xn);
-  if (pending)
-    k_mf_norm<kPartRanges><<<d.batch, 256, 0, stream>>>(st.done, h, w, y, d.hidden, d.rms_eps, sc.mf_part, d.batch);
-  else
-    k_mf_norm<0><<<d.batch, 256, 0, stream>>>(st.done, h, w, y, d.hidden, d.rms_eps, nullptr, d.batch);
+static MfNormArgs norm_args(const KernelEnv& env, const StepPtrs& st, size_t w_off) {
+  MfNormArgs n{};
+  n.done = st.done;
+  n.h = static_cast<bf16_t*>(env.scratch.hidden);
+  n.w = reinterpret_cast<const bf16_t*>(env.weights + w_off);
+  n.y = static_cast<bf16_t*>(env.scratch.xn);
+  n.eps = env.dims.rms_eps;
+  n.part = env.scratch.mf_part;
+  n.B = env.dims.batch;
+  return n;
+}
+
+// The RMSNorm launch after an o or down projection, whose partials it adds.
+static void mf_norm(const KernelEnv& env, const StepPtrs& st, size_t w_off, hipStream_t stream) {
+  k_mf_norm<kPartRanges, false><<<env.dims.batch, kNormThreads, 0, stream>>>(norm_args(env, st, w_off));
 }
 
 hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, int layer, hipStream_t stream) {
@@ -740,7 +782,7 @@ hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, i
   auto pk = [&](size_t off) { return reinterpret_cast<const bf16_t*>(env.packed + off); };
   if (op == MfmaOp::kLmHead) {
     // the last layer's down projection is still in partials
-    mf_norm(env, st, env.final_norm_off, true, stream);
+    mf_norm(env, st, env.final_norm_off, stream);
     a.x = static_cast<const bf16_t*>(sc.xn);
     a.p0 = pk(env.packed_lm_off);
     a.K = d.hidden;
@@ -760,9 +802,24 @@ hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, i
   const PackedOffsets& po = env.packed_off[layer];
   const size_t cache_layer_elems = (size_t)d.slots() * d.kv_dim();
   switch (op) {
+    case MfmaOp::kEmbed: {
+      MfNormArgs n = norm_args(env, st, lo.input_norm);
+      n.token = st.token;
+      n.pos = st.pos;
+      n.embedding = wt(env.embedding_off);
+      n.inv_freq = sc.inv_freq;
+      n.rope = sc.rope;
+      n.active = st.active;
+      n.next_pos = st.next_pos;
+      n.V = d.vocab;
+      n.half = d.head_dim / 2;
+      k_mf_norm<0, true><<<d.batch, kNormThreads, 0, stream>>>(n);
+      break;
+    }
     case MfmaOp::kQkv: {
-      // layer > 0: the previous layer's down projection is still in partials
-      mf_norm(env, st, lo.input_norm, layer > 0, stream);
+      // the previous layer's down projection is still in partials; the first
+      // layer's norm ran with the embedding
+      if (layer > 0) mf_norm(env, st, lo.input_norm, stream);
       a.x = static_cast<const bf16_t*>(sc.xn);
       a.p0 = pk(po.qkv);
       a.w1 = wt(lo.qkv_b);
@@ -797,7 +854,7 @@ hipError_t launch_mfma_op(MfmaOp op, const KernelEnv& env, const StepPtrs& st, i
                                                                                          stream);
       break;
     case MfmaOp::kGateUp:
-      mf_norm(env, st, lo.post_norm, true, stream);
+      mf_norm(env, st, lo.post_norm, stream);
       a.x = static_cast<const bf16_t*>(sc.xn);
       a.p0 = pk(po.gate);
       a.p1 = pk(po.up);

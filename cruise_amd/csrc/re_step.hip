@@ -803,7 +803,11 @@ static hipError_t decoder_step_t(const KernelEnv& env, const StepPtrs& st, hipSt
     ++op;
     return w;
   };
-  if (want()) {
+  const bool embed = want();
+  if (embed && p.mfma) {
+    const hipError_t err = launch_mfma_op(MfmaOp::kEmbed, env, st, 0, stream);
+    if (err != hipSuccess) return err;
+  } else if (embed) {
     EmbedArgs e{};
     e.done = st.done;
     e.token = st.token;
