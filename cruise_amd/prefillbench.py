@@ -10,7 +10,8 @@ rows x (len - 1) tokens through every layer.  Reported per call: wall time,
 tokens/s, and the algorithmic FLOP rate against MI355X's dense bf16 MFMA
 peak (2.5 PFLOP/s): 2 x 233,046,016 linear parameters per token per layer
 plus the causal attention's 4 x (position + 1) x head_dim x heads per token
-per layer (Q K^T and P V).
+per layer (Q K^T and P V).  The last layer counts its key and value
+projections alone, all that a prefill needs of it.
 """
 from __future__ import annotations
 
@@ -21,13 +22,14 @@ import time
 import numpy as np
 
 LINEAR_PARAMS_PER_LAYER = 233_046_016  # q/k/v, o, gate, up, down of Qwen2.5-7B
+KV_PARAMS = 2 * 512 * 3584  # the key and value projections of a layer
 MFMA_BF16_PEAK = 2.5e15
 
 
 def prefill_flops(rows: int, length: int, layers: int, heads: int = 28, head_dim: int = 128) -> float:
     tokens = rows * (length - 1)
     attn = sum(4 * (p + 1) * head_dim * heads for p in range(length - 1)) * rows
-    return float(layers) * (2.0 * LINEAR_PARAMS_PER_LAYER * tokens + attn)
+    return (layers - 1.0) * (2.0 * LINEAR_PARAMS_PER_LAYER * tokens + attn) + 2.0 * KV_PARAMS * tokens
 
 
 def main(argv=None) -> None:
