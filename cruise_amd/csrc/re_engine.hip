@@ -1434,6 +1434,21 @@ extern "C" int32_t resident_epoch_prefill(void* engine, int32_t row, int32_t gen
 
 namespace {
 
+// Waits for the stream when it goes out of scope, so that nothing queued still
+// reads a host buffer declared before it or scratch whose lock is released
+// after it.
+struct StreamWait {
+  hipStream_t stream;
+  bool pending = true;
+  bool finish() {
+    pending = false;
+    return hipStreamSynchronize(stream) == hipSuccess;
+  }
+  ~StreamWait() {
+    if (pending) (void)hipStreamSynchronize(stream);
+  }
+};
+
 // One pass of the decoder over the prompt tokens of several rows (see
 // resident_epoch_prefill_batch).  Token i of the pass is (row, position);
 // a row's tokens are consecutive and start at position 0.
@@ -1514,6 +1529,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   stage(o_slot, slot);
   stage(o_tiles, tiles);
   stage(o_blocks, tables);
+  StreamWait wait{s};  // on every exit from here on: `up` and the scratch are in use
   if (hipMemcpyAsync(b + o_tok, up.data(), tables_bytes, hipMemcpyHostToDevice, s) != hipSuccess) return -2;
   const KernelEnv env = e.env();
   if (launch_clear_blocks(env, e.key_cache, e.value_cache, reinterpret_cast<const int32_t*>(b + o_blocks),
@@ -1625,8 +1641,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   for (int i = 0; i < nr; ++i)
     records.push_back(RowRecord{prompts[i].back(), rows[i], gens[i], static_cast<int32_t>(prompts[i].size())});
   const bool stored = store_rows(e, records);
-  if (hipStreamSynchronize(s) != hipSuccess || !stored) return -2;
-  return 0;
+  return wait.finish() && stored ? 0 : -2;
 }
 
 }  // namespace
