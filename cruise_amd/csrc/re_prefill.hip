@@ -640,12 +640,14 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
 //
 // SwiGLU: W the gate rows, W2 the up rows, out = silu(gate) * up.
 template <int EPI, int MT, bool VEC>
-__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN) {
+__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN, int tiles) {
+  const int tile = blockIdx.y * gridDim.x + blockIdx.x;
+  if (tile >= tiles) return;  // past the last tile of the grid's last row
   constexpr int kT = 16 * MT, kOps = EPI == kGemmSwiGlu ? 2 : 1, kLd = kT + 4;
   constexpr int UN = MT == 1 ? 4 : 2;
   __shared__ __align__(16) float red[4][kOps][kT][kLd];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
-  const int m0 = blockIdx.x / nN * kT, n0 = blockIdx.x % nN * kT;
+  const int m0 = tile / nN * kT, n0 = tile % nN * kT;
   const int fr = lane & 15, fq = lane >> 4;
   // Rows past M or N read a valid row (clamped) whose results are never stored.
   const float* arow[MT];
@@ -1222,14 +1224,18 @@ static hipError_t gemm_f32_launch(const GemmArgs& a, hipStream_t stream) {
   constexpr long long kLargeTiles = 2 * 256;
   auto tiles = [&](int t) { return (long long)((a.M + t - 1) / t) * ((a.N + t - 1) / t); };
   const bool large = tiles(32) >= kLargeTiles;
-  const long long grid = tiles(large ? 32 : 16);
-  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  const long long total = tiles(large ? 32 : 16);
+  // a launch dimension holds fewer than 2^32 threads (more run cut short,
+  // without an error): rows of 2^22 workgroups
+  constexpr long long kGridRow = 1 << 22;
+  if (total > INT32_MAX - kGridRow) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(std::min(total, kGridRow)), static_cast<unsigned>((total + kGridRow - 1) / kGridRow));
   const int nN = (a.N + (large ? 31 : 15)) / (large ? 32 : 16);
   const uintptr_t addr = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W) |
                          (EPI == kGemmSwiGlu ? reinterpret_cast<uintptr_t>(a.W2) : 0);
   const bool vec = (addr & 15) == 0 && a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0;
   auto run = [&](auto mt, auto v) {
-    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<static_cast<unsigned>(grid), 256, 0, stream>>>(a, nN);
+    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<grid, 256, 0, stream>>>(a, nN, static_cast<int>(total));
     return hipGetLastError();
   };
   using one = std::integral_constant<int, 1>;

@@ -6,6 +6,7 @@ four waves) on the GPU.
   against the product in 64 bits.  Each output is K products and K + 2 sums in
   fp32 (the bias or residual one of them), so it is within
   (K + 3) 2^-24 (sum |a| |w| + |bias or residual|) of it in any order.
+* More tiles than one grid dimension holds.
 * The SwiGLU epilogue at both tile sizes: prompts of a small fp32 model
   prefilled together (2,036 tokens: 32 x 32 tiles; 20 tokens: 16 x 16) against
   the engine's own single-row prefill at the model tolerance.
@@ -66,3 +67,21 @@ def test_fp32_swiglu_prefill_matches_single_row_prefill(length):
         check_caches(W, v, v_ref, slots, "values")
     finally:
         rt.close()
+
+
+def test_fp32_gemm_of_more_threads_than_one_grid_dimension_holds(lib):  # noqa: F811
+    """4,097 x 4,097 tiles of 32 x 32: at 256 threads each more than the 2^32 - 1
+    that one dimension of a launch takes; a larger one runs cut short, without
+    an error.  Integer operands: the sums are exact."""
+    M = N = 131_080
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    mk = lambda *s: torch.randint(-8, 9, s, generator=gen, device="cuda").float()
+    A, W = mk(M, 4), mk(N, 4)
+    out = torch.empty(M, N, device="cuda")
+    out[-64:] = -1.0
+    torch.cuda.synchronize()
+    assert run(lib, A, W, None, None, out, 0) == 0
+    for r0 in (0, 64, 4096, 65504, 131_008, M - 40):
+        assert torch.equal(out[r0:r0 + 40], A[r0:r0 + 40] @ W.T), f"rows from {r0}"
+    del out
+    torch.cuda.empty_cache()
