@@ -1926,7 +1926,7 @@ extern "C" int32_t resident_epoch_gemm(const void* A, const void* W, const void*
   using namespace re;
   if (A == nullptr || W == nullptr || out == nullptr || M < 0 || N <= 0 || K <= 0 || epilogue < kGemmStore ||
       epilogue > kGemmSwiGlu || (dtype_bytes != 2 && dtype_bytes != 4) ||
-      (epilogue == kGemmSwiGlu && (W2 == nullptr || dtype_bytes != 2)))
+      (epilogue == kGemmSwiGlu && (W2 == nullptr || (dtype_bytes != 2 && M > 0))))
     return -1;
   // the bf16 kernel reads the bias four elements at a time
   if (dtype_bytes == 2 && epilogue == kGemmStore && bias != nullptr && (reinterpret_cast<uintptr_t>(bias) & 7) != 0)

@@ -23,7 +23,7 @@ from oracle.decoder import PagedGeometry
 from oracle.weights import generate_weights
 from oracle.workloads import C1, random_tables
 from parity import make_runtime
-from test_gpu_gemm import lib, operands, run  # noqa: F401
+from test_gpu_gemm import lib, operands, ptr, run  # noqa: F401
 from test_gpu_prefill import check_caches, read_caches, reset, written_slots
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +85,11 @@ def test_fp32_gemm_of_more_threads_than_one_grid_dimension_holds(lib):  # noqa: 
         assert torch.equal(out[r0:r0 + 40], A[r0:r0 + 40] @ W.T), f"rows from {r0}"
     del out
     torch.cuda.empty_cache()
+
+
+def test_fp32_swiglu_is_refused_and_no_rows_are_not(lib):  # noqa: F811
+    A, W = torch.zeros(1, 8, device="cuda"), torch.zeros(8, 8, device="cuda")
+    out = torch.full((1, 8), 7.0, device="cuda")
+    assert run(lib, A, W, W, None, out, 2) == -1
+    assert lib.resident_epoch_gemm(ptr(A), ptr(W), ptr(W), None, ptr(out), 0, 8, 8, 2, 4) == 0
+    assert bool((out == 7.0).all())
