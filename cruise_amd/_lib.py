@@ -98,6 +98,10 @@ SIGNATURES: dict[str, tuple] = {
         ctypes.c_int32,
         [ctypes.c_void_p] * 5 + [ctypes.c_int32] * 5,
     ),
+    "resident_epoch_gemm_tiled": (
+        ctypes.c_int32,
+        [ctypes.c_void_p] * 5 + [ctypes.c_int32] * 7,
+    ),
 }
 
 _LIB: ctypes.CDLL | None = None

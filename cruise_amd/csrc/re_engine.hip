@@ -1499,7 +1499,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
   const size_t rows_bytes = off, tables_bytes = o_blocks + 4 * tables.size() - o_tok;
   // K ranges of the qkv, o and down GEMMs (bf16); each one's partial sums are
   // consumed before the next writes its own
-  auto plan_of = [&](int N, int K) { return T == 2 && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{4, 1}; };
+  auto plan_of = [&](int N, int K) { return T == 2 && M > 0 ? plan_gemm(M, N, K, false, kPrefillPartBytes) : GemmPlan{}; };
   const GemmPlan qkv_plan = plan_of(d.qkv_rows(), d.hidden), o_plan = plan_of(d.hidden, d.q_dim()),
                  down_plan = plan_of(d.hidden, d.intermediate), kv_plan = plan_of(2 * d.kv_dim(), d.hidden);
   size_t part_bytes = 0;
@@ -1557,7 +1557,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
       const LayerOffsets& lo = e.layer_off[l];
       float* part = reinterpret_cast<float*>(b + o_part);
       auto gemm = [&](size_t a_off, long long lda, size_t w_off, size_t bias_off, size_t out_off, long long ldo, int N,
-                      int K, int epi, GemmPlan plan = {4, 1}) {
+                      int K, int epi, GemmPlan plan) {
         GemmArgs g{};
         g.A = b + a_off;
         g.W = e.weights + w_off;
@@ -1577,7 +1577,7 @@ int32_t prefill_batch(Engine& e, const std::vector<int>& rows, const std::vector
         run(launch_prefill_rmsnorm(b + o_hidden, e.weights + w_off, b + o_xn, M, d.hidden, d.rms_eps, d.dtype_bytes, part,
                                    before.splits > 1 ? before.splits : 0, s));
       };
-      norm(lo.input_norm, l > 0 ? down_plan : GemmPlan{4, 1});
+      norm(lo.input_norm, l > 0 ? down_plan : GemmPlan{});
       // Nothing reads what the last layer computes past its keys and values
       // (the first decode step starts from the prompt's last token), so it
       // stops there: the k and v rows of the stacked projection, as a matrix
@@ -1921,6 +1921,34 @@ extern "C" int32_t resident_epoch_time_layer_op(void* engine, int32_t which, int
   return 0;
 }
 
+namespace {
+// A GEMM of caller buffers with packed rows, on the null stream.
+int32_t gemm_call(const void* A, const void* W, const void* W2, const void* bias, void* out, int M, int N, int K,
+                  int epilogue, int dtype_bytes, re::GemmPlan plan) {
+  using namespace re;
+  GemmArgs g{};
+  g.A = A;
+  g.W = W;
+  g.W2 = W2;
+  g.out = out;
+  g.bias = epilogue == kGemmStore ? bias : nullptr;
+  if (epilogue == kGemmPart) g.part = static_cast<float*>(out);
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.lda = K;
+  g.ldw = K;
+  g.ldo = N;
+  const hipError_t e = launch_gemm(g, epilogue, dtype_bytes, nullptr, plan);
+  if (e == hipErrorInvalidValue) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (e != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) return -2;
+  return 0;
+}
+}  // namespace
+
 extern "C" int32_t resident_epoch_gemm(const void* A, const void* W, const void* W2, const void* bias, void* out,
                                        int32_t M, int32_t N, int32_t K, int32_t epilogue, int32_t dtype_bytes) {
   using namespace re;
@@ -1931,25 +1959,23 @@ extern "C" int32_t resident_epoch_gemm(const void* A, const void* W, const void*
   // the bf16 kernel reads the bias four elements at a time
   if (dtype_bytes == 2 && epilogue == kGemmStore && bias != nullptr && (reinterpret_cast<uintptr_t>(bias) & 7) != 0)
     return -1;
-  GemmArgs g{};
-  g.A = A;
-  g.W = W;
-  g.W2 = W2;
-  g.out = out;
-  g.bias = epilogue == kGemmStore ? bias : nullptr;
-  g.M = M;
-  g.N = N;
-  g.K = K;
-  g.lda = K;
-  g.ldw = K;
-  g.ldo = N;
-  const hipError_t e = launch_gemm(g, epilogue, dtype_bytes, nullptr);
-  if (e == hipErrorInvalidValue) {
-    (void)hipGetLastError();
+  return gemm_call(A, W, W2, bias, out, M, N, K, epilogue, dtype_bytes, GemmPlan{});
+}
+
+extern "C" int32_t resident_epoch_gemm_tiled(const void* A, const void* W, const void* W2, const void* bias, void* out,
+                                             int32_t M, int32_t N, int32_t K, int32_t epilogue, int32_t dtype_bytes,
+                                             int32_t tile_rows, int32_t ranges) {
+  using namespace re;
+  if (A == nullptr || W == nullptr || out == nullptr || M < 0 || N <= 0 || K <= 0 || epilogue < kGemmStore ||
+      epilogue > kGemmPart || (dtype_bytes != 2 && dtype_bytes != 4) || (epilogue == kGemmSwiGlu && W2 == nullptr))
     return -1;
-  }
-  if (e != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) return -2;
-  return 0;
+  if (dtype_bytes == 4 ? epilogue == kGemmPart || tile_rows != 0 || ranges != 1
+                       : tile_rows < 64 || tile_rows > 256 || tile_rows % 64 != 0 || ranges < 1 ||
+                             (ranges > 1 && epilogue != kGemmPart))
+    return -1;
+  if (dtype_bytes == 2 && epilogue == kGemmStore && bias != nullptr && (reinterpret_cast<uintptr_t>(bias) & 7) != 0)
+    return -1;
+  return gemm_call(A, W, W2, bias, out, M, N, K, epilogue, dtype_bytes, GemmPlan{tile_rows / 64, ranges});
 }
 
 extern "C" int32_t resident_epoch_kernel_timing(void* engine, int32_t enable) {

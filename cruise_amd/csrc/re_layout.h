@@ -315,9 +315,9 @@ struct PrefillAttn {           // causal attention within each row's prompt
 // T(T(silu(T(gate))) * T(up)) over N output columns.
 // Part (bf16 only): the fp32 partial sums of K ranges, to part.
 enum GemmEpilogue : int { kGemmStore = 0, kGemmResidual = 1, kGemmSwiGlu = 2, kGemmPart = 3 };
-// Tile rows (64 mj) and K ranges of a bf16 GEMM (plan_gemm).
+// Tile rows (64 mj) and K ranges of a bf16 GEMM (plan_gemm); mj 0: not chosen.
 struct GemmPlan {
-  int mj, splits;
+  int mj = 0, splits = 1;
 };
 struct GemmArgs {              // out[M,N] (epilogue) A[M,K] W[N,K]^T
   const void* A;
@@ -335,10 +335,10 @@ hipError_t launch_prefill_rmsnorm(void* x, const void* w, void* y, int M, int H,
                                   const float* part, int parts, hipStream_t stream);
 hipError_t launch_prefill_qkv_post(const PrefillQkv& a, int dtype_bytes, hipStream_t stream);
 // The fastest tile and K ranges for a shape whose partial sums take at most
-// part_bytes; launch_gemm follows `plan` when a.part is set, else it picks the
-// tile itself and runs one K range.
+// part_bytes; launch_gemm follows `plan` (more than one range: with a.part
+// set), or picks the tile of a single range itself.
 GemmPlan plan_gemm(int M, int N, int K, bool swiglu, size_t part_bytes);
-hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream, GemmPlan plan = {4, 1});
+hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t stream, GemmPlan plan = {});
 // The MFMA attention serves bf16 models with head_dim 128 (64-query tiles).
 bool prefill_attention_mfma(const Dims& d);
 size_t prefill_attention_lds(const Dims& d, int max_keys);

@@ -1288,8 +1288,9 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int dtype_bytes, hipStream_t 
     if (a.K <= 0 || a.K % kGk != 0 || a.N % 8 != 0 || a.lda % 8 != 0 || a.ldw % 8 != 0 || a.ldo % 8 != 0 ||
         !aligned || (swiglu && a.W2 == nullptr))
       return hipErrorInvalidValue;
-    const GemmPlan p = a.part != nullptr ? plan : plan_gemm(a.M, a.N, a.K, swiglu, 0);
-    if (p.mj < 1 || p.mj > 4 || p.splits < 1 || p.splits > a.K / kGk) return hipErrorInvalidValue;
+    const GemmPlan p = plan.mj != 0 ? plan : plan_gemm(a.M, a.N, a.K, swiglu, 0);
+    if (p.mj < 1 || p.mj > 4 || p.splits < 1 || p.splits > a.K / kGk || (p.splits > 1 && a.part == nullptr))
+      return hipErrorInvalidValue;
     if (a.part != nullptr) return gemm_launch_mj<kGemmPart>(a, p, stream);
     if (epi == kGemmStore) return gemm_launch_mj<kGemmStore>(a, p, stream);
     if (epi == kGemmResidual) return gemm_launch_mj<kGemmResidual>(a, p, stream);

@@ -249,6 +249,17 @@ int32_t resident_epoch_time_layer_op(void *engine, int32_t which, int32_t passes
 int32_t resident_epoch_gemm(const void *A, const void *W, const void *W2, const void *bias, void *out,
                             int32_t M, int32_t N, int32_t K, int32_t epilogue, int32_t dtype_bytes);
 
+/* The same products on a given tile, for checking every tile height and every
+ * split of K that a prefill may choose.  bf16: tile_rows 64, 128, 192 or 256;
+ * epilogue 3 cuts K into `ranges` (1 to K / 64) runs of whole 64-element steps,
+ * range r the steps from r (K / 64) / ranges, rounded down, to the next one's,
+ * and writes their fp32 sums to out[ranges][M][N]; the other epilogues take
+ * one range.  fp32: epilogues 0 to 2, tile_rows 0 and ranges 1 (the tile
+ * follows from the shape).  Otherwise as resident_epoch_gemm. */
+int32_t resident_epoch_gemm_tiled(const void *A, const void *W, const void *W2, const void *bias, void *out,
+                                  int32_t M, int32_t N, int32_t K, int32_t epilogue, int32_t dtype_bytes,
+                                  int32_t tile_rows, int32_t ranges);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,13 +1,14 @@
 """The batched prefill's GEMM plans (tile height, K ranges) on the GPU.
 
-* every tile height, at heights that leave a partial last tile, against the
-  CPU product: integer operands, so fp32 sums are exact in any order and the
-  store and residual epilogues must agree bit for bit (as in
-  test_gpu_gemm.py, whose shapes take the 64-row tile);
+* products whose planned tiles are 128, 192 and 256 rows high, at heights that
+  leave a partial last tile, against the CPU product: integer operands, so fp32
+  sums are exact in any order and the store and residual epilogues must agree
+  bit for bit (as in test_gpu_gemm.py, whose shapes take the 64-row tile;
+  test_gpu_gemm_tiled.py checks every height whatever the planner chooses);
 * split K: two Qwen2.5-7B layers (the second layer's keys and values go
   through the first one's qkv, o and down partial sums) at token counts
   around the tile edges, against the engine's own single-row prefill at the
-  model tolerance;
+  model tolerance (test_gpu_prefill_exact.py: exactly);
 * the no-allocation entry point chooses the same K ranges: equal bits.
 """
 from __future__ import annotations

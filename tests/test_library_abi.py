@@ -181,3 +181,19 @@ def test_gemm_entry_point_rejects_bad_arguments_before_any_device_work(lib):
     assert f(p, p, null, null, p, 8, 8, 64, 0, 3) == -1  # element size
     assert f(p, p, null, null, p, 8, 8, 64, 2, 2) == -1  # SwiGLU without the up rows
     assert f(p, p, null, ctypes.c_void_p(20), p, 8, 8, 64, 0, 2) == -1  # bias not 8-byte aligned
+
+
+def test_tiled_gemm_entry_point_rejects_bad_arguments_before_any_device_work(lib):
+    p = ctypes.c_void_p(16)  # never dereferenced: the checks fail first
+    f = lib.resident_epoch_gemm_tiled
+    assert f(None, p, None, None, p, 8, 8, 64, 0, 2, 64, 1) == -1  # no A
+    assert f(p, p, None, None, p, 8, 8, 64, 4, 2, 64, 1) == -1  # no such epilogue
+    assert f(p, p, None, None, p, 8, 8, 64, 2, 2, 64, 1) == -1  # SwiGLU without the up rows
+    assert f(p, p, None, None, p, 8, 8, 64, 0, 2, 0, 1) == -1  # bf16 tile heights
+    assert f(p, p, None, None, p, 8, 8, 64, 0, 2, 96, 1) == -1
+    assert f(p, p, None, None, p, 8, 8, 64, 0, 2, 320, 1) == -1
+    assert f(p, p, None, None, p, 8, 8, 64, 3, 2, 64, 0) == -1  # ranges
+    assert f(p, p, None, None, p, 8, 8, 128, 0, 2, 64, 2) == -1  # ranges of another epilogue
+    assert f(p, p, None, None, p, 8, 8, 64, 3, 4, 0, 1) == -1  # fp32 partial sums
+    assert f(p, p, None, None, p, 8, 8, 64, 0, 4, 64, 1) == -1  # fp32 on a given tile
+    assert f(p, p, None, ctypes.c_void_p(20), p, 8, 8, 64, 0, 2, 64, 1) == -1  # bias not 8-byte aligned
