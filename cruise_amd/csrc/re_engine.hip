@@ -590,8 +590,10 @@ bool alloc_state(Engine& e) {
 
 // The packed copy of the projections (matrix-core plan).  Below 64 rows it is
 // taken only while the buffers that grow later (the decoder-step caches, a
-// prefill of every row's window) still fit beside it.
-bool alloc_packed(Engine& e) {
+// prefill of every row's window) still fit beside it, and it takes at most
+// "tuning": {"packed_limit": bytes}; otherwise the engine keeps the row-tiled
+// kernels, whose sums run in another order.
+bool alloc_packed(Engine& e, const Json& cfg) {
   if (!e.plan.mfma) return true;
   const Dims& d = e.dims;
   e.packed_off.resize(d.layers);
@@ -600,6 +602,9 @@ bool alloc_packed(Engine& e) {
     const size_t token = (2 * (size_t)d.hidden + d.qkv_rows() + d.q_dim() + d.intermediate) * d.dtype_bytes +
                          (size_t)d.head_dim * sizeof(float) + 64;
     const size_t later = 2 * e.cache_bytes + (size_t)d.batch * d.capacity * token + kPrefillPartBytes + (1ull << 30);
+    const Json* tune = cfg.get("tuning");
+    if (tune != nullptr && static_cast<double>(bytes) > tune->number_or("packed_limit", static_cast<double>(bytes)))
+      return false;
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < bytes + later) return false;
   }
@@ -1060,7 +1065,7 @@ extern "C" void* resident_epoch_create(const char* air_path, const char* graph_c
     *status = kCreateDevice;
     return nullptr;
   }
-  if (!alloc_state(*e) || !alloc_packed(*e)) {
+  if (!alloc_state(*e) || !alloc_packed(*e, cfg)) {
     // without the room for the packed weights below 64 rows: the row-tiled plan
     const bool retry = e->plan.mfma && e->dims.batch < 64;
     free_state(*e);
