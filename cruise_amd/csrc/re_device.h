@@ -274,7 +274,7 @@ __device__ __forceinline__ void wave_reduce_transpose(float (&v)[N], int lane) {
 // Workgroup barrier that orders LDS only.  __syncthreads() also orders global
 // memory, so it waits for every global load in flight; this one lets weight
 // loads issued before it stay in flight across the barrier.
-// Packed 64-row activations of the matrix-core path: row m, element k of a
+// Packed activations of the matrix-core path: row m, element k of a
 // [rows, K] block at ((m/16 * K/32 + k/32) * 64 + (m%16 + 16 (k%32)/8)) * 8 +
 // k%8, so a wave's MFMA fragment of one 16-row tile and one 32-wide k step is
 // 1 KB contiguous (rows a multiple of 16, K of 32).

@@ -302,9 +302,14 @@ bool make_plan(Engine& e, const Json& cfg, bool packed) {
   // row-tiled kernels, and so does an engine without the memory for the
   // packed weights.  The row-tiled kernels read every weight once per 8 rows:
   // a step of one layer and the LM head at 16 rows took 600 us there and
-  // takes 312 here, two layers and the head at 41 rows 2,229 and 481.  At up
-  // to four rows the four-row kernels stream the weights once and need no
-  // partial sums.
+  // takes 312 here, two layers and the head at 41 rows 2,229 and 481.  At 5 to
+  // 8 rows both read them once, and the products are what is saved: an epoch
+  // of eight steps of one layer and the head takes 2,325-2,360 us here and
+  // 2,428-2,553 there, of four layers 5,037-5,066 and 5,438-5,556.  At up to
+  // four rows the four-row kernels stream the weights once and need no partial
+  // sums.  The packed weights are a second copy of the projections, 0.47 GB a
+  // layer and 1.09 GB for the head; an engine that would rather have the
+  // memory asks for "mfma": 0.
   p.mfma = 0;
   p.gu_cu = 0;
   if (packed && mfma_step_supported(d) && mfma_lm_cu_fits(d, e.cus) && mfma_gu_cu_fits(d, e.cus) && mfma_qkv_split_fits(d) &&

@@ -155,7 +155,7 @@ struct LaunchPlan {
   // Down projection with the whole K in one workgroup (re_step.hip
   // k_down_whole): 0 = split-K segments + reduce launch; else its grid.
   int down_whole_grid;
-  // 1: the projections run on the matrix cores (re_mfma.hip, 64 rows)
+  // 1: the projections run on the matrix cores (re_mfma.hip, 5 to 64 rows)
   int mfma;
   // > 0 (with mfma): gate/up runs one workgroup per CU (k_mf_gu_cu), this grid
   int gu_cu;
@@ -229,7 +229,7 @@ bool layer_op_launches(const KernelEnv& env, int which);
 int timed_op_index(const KernelEnv& env, int layer);
 // Grid sizes of the grid-stride projections from the kernels' occupancy.
 void plan_grids(LaunchPlan& p, const Dims& d, int cus);
-// Decode projections on the matrix cores at 64 batch rows (re_mfma.hip):
+// Decode projections on the matrix cores at 5 to 64 batch rows (re_mfma.hip):
 // the RMSNorm (where the projection has one) and the projection of one op.
 enum class MfmaOp { kEmbed, kQkv, kO, kGateUp, kDown, kLmHead };
 bool mfma_step_supported(const Dims& d);

@@ -117,7 +117,11 @@ int32_t resident_epoch_proc(void *engine, const void *feed, int64_t feed_bytes,
  * key_cache/value_cache (host or device) are read and updated in place; the
  * other inputs are host or device arrays of B rows; logits (fp32 [B,V]) and
  * next_position (i64[B]) are written (host or device).  The engine's resident
- * epoch state is not touched.  Return 0, -1 bad arguments, -2 HIP failure. */
+ * epoch state is not touched.  Return 0, -1 bad arguments, -2 HIP failure.
+ * The kernels work on 16-byte aligned caches in the engine's device memory
+ * directly: a step that fails (-2) may leave the slots that it addresses
+ * written in them, every other byte as it was (a repeated step writes the same
+ * slots).  Other caches are copied back only once the step has run. */
 int32_t resident_decoder_step(void *engine, const int64_t *token_id,
                               const int64_t *position,
                               const int32_t *sequence_length, void *key_cache,
