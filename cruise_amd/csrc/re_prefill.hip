@@ -623,6 +623,11 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   }
 }
 
+// The fp32 kernel's tiles are numbered through rows of 2^22 workgroups: a launch
+// dimension holds fewer than 2^32 threads (more run cut short, without an
+// error).  Workgroups past the last tile have only rows past M.
+constexpr int kF32GridRow = 1 << 22;
+
 // fp32 models: one 16 MT x 16 MT output tile per workgroup of four waves, on
 // v_mfma_f32_16x16x4_f32 (fp32 operands and sums).  K goes to the waves in
 // 16-element chunks, chunk c to wave c % 4, so the workgroup reads its rows in
@@ -644,13 +649,12 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
 //
 // SwiGLU: W the gate rows, W2 the up rows, out = silu(gate) * up.
 template <int EPI, int MT, bool VEC>
-__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN, int tiles) {
-  const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-  if (tile >= tiles) return;  // past the last tile of the grid's last row
+__global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN) {
   constexpr int kT = 16 * MT, kOps = EPI == kGemmSwiGlu ? 2 : 1, kLd = kT + 4;
   constexpr int UN = MT == 1 ? 4 : 2;
   __shared__ __align__(16) float red[4][kOps][kT][kLd];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
+  const int tile = blockIdx.y * kF32GridRow + blockIdx.x;
   const int m0 = tile / nN * kT, n0 = tile % nN * kT;
   const int fr = lane & 15, fq = lane >> 4;
   // Rows past M or N read a valid row (clamped) whose results are never stored.
@@ -1231,17 +1235,17 @@ static hipError_t gemm_f32_launch(const GemmArgs& a, hipStream_t stream) {
   auto tiles = [&](int t) { return (long long)((a.M + t - 1) / t) * ((a.N + t - 1) / t); };
   const bool large = tiles(32) >= kLargeTiles;
   const long long total = tiles(large ? 32 : 16);
-  // a launch dimension holds fewer than 2^32 threads (more run cut short,
-  // without an error): rows of 2^22 workgroups
-  constexpr long long kGridRow = 1 << 22;
-  if (total > INT32_MAX - kGridRow) return hipErrorInvalidValue;
-  const dim3 grid(static_cast<unsigned>(std::min(total, kGridRow)), static_cast<unsigned>((total + kGridRow - 1) / kGridRow));
   const int nN = (a.N + (large ? 31 : 15)) / (large ? 32 : 16);
+  // tile numbers and row numbers, those past M included, are 32-bit
+  if (total > INT32_MAX - kF32GridRow || (total + kF32GridRow) / nN * (large ? 32 : 16) > INT32_MAX - 64)
+    return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(std::min<long long>(total, kF32GridRow)),
+                  static_cast<unsigned>((total + kF32GridRow - 1) / kF32GridRow));
   const uintptr_t addr = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W) |
                          (EPI == kGemmSwiGlu ? reinterpret_cast<uintptr_t>(a.W2) : 0);
   const bool vec = (addr & 15) == 0 && a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0;
   auto run = [&](auto mt, auto v) {
-    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<grid, 256, 0, stream>>>(a, nN, static_cast<int>(total));
+    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<grid, 256, 0, stream>>>(a, nN);
     return hipGetLastError();
   };
   using one = std::integral_constant<int, 1>;
