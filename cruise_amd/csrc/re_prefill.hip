@@ -1339,6 +1339,10 @@ hipError_t launch_prefill_attention(const PrefillAttn& a, const Dims& d, int nti
   if (prefill_attention_mfma(d)) {
     if (ntiles <= 0) return hipErrorInvalidValue;
     if (d.heads % d.kv_heads != 0) return hipErrorInvalidValue;
+    // The pass's longest prompt decides for all of its rows: one of more than
+    // 1,024 tokens has the shorter ones compute their scores twice too, as every
+    // prompt would without the kept scores (64 rows of 999 tokens, a layer:
+    // 2,100 us against 1,497).
     const int grid = flash_grid(ntiles, d.heads, d.kv_heads), key_tiles = (a.max_keys + kAk - 1) / kAk;
     if (key_tiles <= 1)
       k_pf_attn_flash<1><<<grid, 256, 0, stream>>>(a, ntiles);
