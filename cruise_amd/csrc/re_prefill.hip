@@ -14,7 +14,8 @@
 //              where the tiles alone leave CUs idle, the partial sums added
 //              by the row kernel that follows.  fp32 models: 16 x 16 and
 //              32 x 32 tiles on the fp32 MFMA, K split over a workgroup's
-//              waves, the same epilogues.
+//              waves; 64 x 64 tiles through LDS on the vector units for large
+//              products; the same epilogues.
 //   qkv post   RoPE of q and k in place, K/V rows to their paged slots
 //   attention  causal within each row's prompt.  bf16, head_dim 128: MFMA
 //              for Q K^T and P V per (64-query tile, head), the softmax the
@@ -623,12 +624,74 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
   }
 }
 
-// The fp32 kernel's tiles are numbered through rows of 2^22 workgroups: a launch
-// dimension holds fewer than 2^32 threads (more run cut short, without an
-// error).  Workgroups past the last tile have only rows past M.
-constexpr int kF32GridRow = 1 << 22;
+// fp32 models, large products: 64 x 64 tiles through LDS on the vector units, 4
+// x 4 sums per thread, K in steps of 16.  SwiGLU: 32 output columns, in LDS two
+// gate rows and their two up rows in turn, so a thread's four sums of a row are
+// gate and up of two columns and the launch has as many workgroups as the two
+// products.  Bound by the vector units' rate and LDS reads, 70-77 TFLOP/s;
+// the matrix-core kernel below reads its operands from L2 for every 32 x 32 tile
+// and stays at 60 (22-27 where it has to load element by element).  See
+// gemm_f32_launch.  m_on_x: the grid's first dimension runs over M tiles, else
+// over N tiles.
+template <int EPI>
+__global__ void __launch_bounds__(256) k_gemm_f32_lds(GemmArgs a, int m_on_x) {
+  constexpr bool kSwiGlu = EPI == kGemmSwiGlu;
+  constexpr int kTileN = kSwiGlu ? 32 : 64;
+  __shared__ float As[16][64 + 4];
+  __shared__ float Ws[16][64 + 4];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int m0 = (m_on_x ? blockIdx.x : blockIdx.y) * 64, n0 = (m_on_x ? blockIdx.y : blockIdx.x) * kTileN;
+  const float* A = static_cast<const float*>(a.A);
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < a.K; k0 += 16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // rows past M or N read a valid row (clamped) whose results are never stored
+      const int idx = tid + 256 * i, row = idx >> 4, kk = idx & 15, k = k0 + kk;
+      const bool kin = k < a.K;
+      const float* W = static_cast<const float*>(kSwiGlu && i >= 2 ? a.W2 : a.W);  // rows 32.. from i = 2 on
+      const float x = A[(size_t)min(m0 + row, a.M - 1) * a.lda + (kin ? k : 0)];
+      const float y = W[(size_t)min(n0 + row % kTileN, a.N - 1) * a.ldw + (kin ? k : 0)];
+      As[kk][row] = kin ? x : 0.f;
+      Ws[kk][kSwiGlu ? (row % 32 / 2) * 4 + (row / 32) * 2 + row % 2 : row] = kin ? y : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+      float av[4], wv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        av[r] = As[kk][ty * 4 + r];
+        wv[r] = Ws[kk][tx * 4 + r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[r][c] = fmaf(av[r], wv[c], acc[r][c]);
+    }
+    __syncthreads();
+  }
+  float* out = static_cast<float*>(a.out);
+  const float* bias = static_cast<const float*>(a.bias);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < (kSwiGlu ? 2 : 4); ++c) {
+      const int m = m0 + ty * 4 + r, n = n0 + tx * (kSwiGlu ? 2 : 4) + c;
+      if (m >= a.M || n >= a.N) continue;
+      float* o = out + (size_t)m * a.ldo + n;
+      const float y = acc[r][c];
+      if constexpr (EPI == kGemmStore)
+        *o = y + (bias != nullptr ? bias[n] : 0.f);
+      else if constexpr (EPI == kGemmResidual)
+        *o = *o + y;
+      else
+        *o = y / (1.0f + expf(-y)) * acc[r][c + 2];
+    }
+}
 
-// fp32 models: one 16 MT x 16 MT output tile per workgroup of four waves, on
+// fp32 models, smaller products: one 16 MT x 16 MT output tile per workgroup of
+// four waves, on
 // v_mfma_f32_16x16x4_f32 (fp32 operands and sums).  K goes to the waves in
 // 16-element chunks, chunk c to wave c % 4, so the workgroup reads its rows in
 // contiguous 256-byte pieces; a lane takes four consecutive K elements of its
@@ -654,8 +717,7 @@ __global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs a, int nN) {
   constexpr int UN = MT == 1 ? 4 : 2;
   __shared__ __align__(16) float red[4][kOps][kT][kLd];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(tid);
-  const int tile = blockIdx.y * kF32GridRow + blockIdx.x;
-  const int m0 = tile / nN * kT, n0 = tile % nN * kT;
+  const int m0 = blockIdx.x / nN * kT, n0 = blockIdx.x % nN * kT;
   const int fr = lane & 15, fq = lane >> 4;
   // Rows past M or N read a valid row (clamped) whose results are never stored.
   const float* arow[MT];
@@ -1224,28 +1286,41 @@ static hipError_t gemm_launch_mj(const GemmArgs& a, const GemmPlan& p, hipStream
   }
 }
 
-// 32 x 32 tiles (twice the products per byte) where they still are two
-// workgroups per CU, else 16 x 16.  Both measured (M x N x K, 16 x 16 against
-// 32 x 32): 66 x 256 x 688 5.0 and 8.9 us, 500 x 256 x 688 6.8 and 9.2, 500 x
-// 512 x 256 6.7 and 6.0; 2,044 x 256 x 688 20.0 and 15.6, 2,044 x 1,376 x 256
-// 44.0 and 31.2, 8,000 x 512 x 256 61.2 and 43.1.
+// Three kernels by the number of tiles, so that each still gives every CU work:
+// - through LDS from four tiles per CU on, where both operands can be read 16
+//   bytes at a time, else past one per CU.  Matrix cores and LDS (M x N x K):
+//   1,000 x 3,584 x 1,024 (896 tiles) 140 and 147 us, 2,000 x 2,048 x 1,024
+//   (1,024) 155 and 149, 4,096 x 4,096 x 1,024 (4,096) 597 and 487; 4-byte
+//   loads, 1,000 x 1,000 x 1,023 (256) 95 and 110, 1,024 x 1,536 x 1,023 (384)
+//   143 and 109, 4,096 x 4,096 x 1,023 1,413 and 503.  SwiGLU: 512 x 3,584 x
+//   1,024 (896) 136 and 142, 1,000 x 2,048 x 1,024 (1,024) 148 and 146, 4,096 x
+//   4,096 x 1,024 1,142 and 934 (two products, the elementwise pass not
+//   counted: 960).
+// - below, on the matrix cores, 32 x 32 (twice the products per byte) from two
+//   workgroups per CU on, else 16 x 16 (16 x 16 against 32 x 32): 66 x 256 x 688
+//   5.0 and 8.9 us, 500 x 256 x 688 6.8 and 9.2, 500 x 512 x 256 6.7 and 6.0;
+//   2,044 x 256 x 688 20.0 and 15.6, 2,044 x 1,376 x 256 44.0 and 31.2.
 template <int EPI>
 static hipError_t gemm_f32_launch(const GemmArgs& a, hipStream_t stream) {
-  constexpr long long kLargeTiles = 2 * 256;
-  auto tiles = [&](int t) { return (long long)((a.M + t - 1) / t) * ((a.N + t - 1) / t); };
-  const bool large = tiles(32) >= kLargeTiles;
-  const long long total = tiles(large ? 32 : 16);
-  const int nN = (a.N + (large ? 31 : 15)) / (large ? 32 : 16);
-  // tile numbers and row numbers, those past M included, are 32-bit
-  if (total > INT32_MAX - kF32GridRow || (total + kF32GridRow) / nN * (large ? 32 : 16) > INT32_MAX - 64)
-    return hipErrorInvalidValue;
-  const dim3 grid(static_cast<unsigned>(std::min<long long>(total, kF32GridRow)),
-                  static_cast<unsigned>((total + kF32GridRow - 1) / kF32GridRow));
+  constexpr unsigned kCus = 256;
+  auto tiles = [&](int t) { return ((long long)a.M + t - 1) / t * (((long long)a.N + t - 1) / t); };
   const uintptr_t addr = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.W) |
                          (EPI == kGemmSwiGlu ? reinterpret_cast<uintptr_t>(a.W2) : 0);
   const bool vec = (addr & 15) == 0 && a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0;
+  constexpr unsigned kTileN = EPI == kGemmSwiGlu ? 32 : 64;
+  const unsigned m_tiles = (a.M + 63u) / 64, n_tiles = (a.N + kTileN - 1) / kTileN;
+  const unsigned long long lds_tiles = (unsigned long long)m_tiles * n_tiles;
+  if (vec ? lds_tiles >= 4 * kCus : lds_tiles > kCus) {
+    // N tiles next to each other share A's rows in L2; a grid's second dimension holds 65,535
+    const int m_on_x = m_tiles > 65535;
+    k_gemm_f32_lds<EPI><<<m_on_x ? dim3(m_tiles, n_tiles) : dim3(n_tiles, m_tiles), 256, 0, stream>>>(a, m_on_x);
+    return hipGetLastError();
+  }
+  const bool large = tiles(32) >= 2 * kCus;
+  const int t = large ? 32 : 16, nN = (a.N + t - 1) / t;
   auto run = [&](auto mt, auto v) {
-    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value><<<grid, 256, 0, stream>>>(a, nN);
+    k_gemm_f32<EPI, decltype(mt)::value, decltype(v)::value>
+        <<<static_cast<unsigned>(tiles(t)), 256, 0, stream>>>(a, nN);
     return hipGetLastError();
   };
   using one = std::integral_constant<int, 1>;

@@ -1,12 +1,12 @@
-"""The fp32 prefill GEMM (fp32 MFMA, 16 x 16 and 32 x 32 tiles, K split over
-four waves) on the GPU.
+"""The fp32 prefill GEMM on the GPU: fp32 MFMA on 16 x 16 and 32 x 32 tiles, K
+split over four waves, and 64 x 64 tiles through LDS for large products.
 
 * Edges of the tiles, of the 16-element K chunks and of the four waves' turns,
-  both tile sizes (32 x 32 from 512 tiles on), aligned and unaligned rows,
-  against the product in 64 bits.  Each output is K products and K + 2 sums in
+  every tile size (32 x 32 from 512 tiles on; 64 x 64 from 1,024 on, unaligned
+  from 257 on), aligned and unaligned rows, against the product in 64 bits.  Each output is K products and K + 2 sums in
   fp32 (the bias or residual one of them), so it is within
   (K + 3) 2^-24 (sum |a| |w| + |bias or residual|) of it in any order.
-* More tiles than one grid dimension holds.
+* More tiles than a grid dimension holds.
 * The SwiGLU epilogue at both tile sizes: prompts of a small fp32 model
   prefilled together (2,036 tokens: 32 x 32 tiles; 20 tokens: 16 x 16) against
   the engine's own single-row prefill at the model tolerance.
@@ -29,7 +29,8 @@ from test_gpu_prefill import check_caches, read_caches, reset, written_slots
 pytestmark = pytest.mark.gpu
 
 SMALL = [(1, 1, 1), (15, 17, 3), (16, 16, 64), (17, 33, 68), (66, 256, 688), (31, 48, 272), (5, 7, 1000)]
-LARGE = [(512, 1024, 16), (496, 1024, 40), (1030, 1041, 33), (2032, 688, 256)]
+LARGE = [(512, 1024, 16), (496, 1024, 40), (1030, 1041, 33), (2032, 688, 256), (1024, 1024, 20), (1025, 1024, 7),
+         (2048, 2048, 36), (1985, 2047, 12), (1984, 2112, 64)]
 
 
 @pytest.mark.parametrize("M,N,K", SMALL + LARGE)
@@ -69,11 +70,11 @@ def test_fp32_swiglu_prefill_matches_single_row_prefill(length):
         rt.close()
 
 
-def test_fp32_gemm_of_more_threads_than_one_grid_dimension_holds(lib):  # noqa: F811
-    """4,097 x 4,097 tiles of 32 x 32: at 256 threads each more than the 2^32 - 1
-    that one dimension of a launch takes; a larger one runs cut short, without
-    an error.  Integer operands: the sums are exact."""
-    M = N = 131_080
+@pytest.mark.parametrize("M,N", [(131_080, 131_080), (4_194_330, 70), (70, 4_194_330)])
+def test_fp32_gemm_of_many_tiles(lib, M, N):  # noqa: F811
+    """69 GB of output: 2^24 tiles of 32 x 32, at 256 threads each more than one
+    grid dimension holds; and more tiles along M or N than a grid's second
+    dimension holds.  Integer operands: the sums are exact."""
     gen = torch.Generator(device="cuda").manual_seed(11)
     mk = lambda *s: torch.randint(-8, 9, s, generator=gen, device="cuda").float()
     A, W = mk(M, 4), mk(N, 4)
@@ -81,8 +82,9 @@ def test_fp32_gemm_of_more_threads_than_one_grid_dimension_holds(lib):  # noqa: 
     out[-64:] = -1.0
     torch.cuda.synchronize()
     assert run(lib, A, W, None, None, out, 0) == 0
-    for r0 in (0, 64, 4096, 65504, 131_008, M - 40):
-        assert torch.equal(out[r0:r0 + 40], A[r0:r0 + 40] @ W.T), f"rows from {r0}"
+    for r0 in (0, 64, 4096, 65504, 131_008, 4_194_250, M - 40):
+        if r0 < M:
+            assert torch.equal(out[r0:r0 + 40], A[r0:r0 + 40] @ W.T), f"rows from {r0}"
     del out
     torch.cuda.empty_cache()
 

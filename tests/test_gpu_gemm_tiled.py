@@ -6,7 +6,7 @@ tile height and every split of K is checked whatever the planner chooses.
   range against the product over that range's columns, bit for bit: ranges of
   one step, of fewer and of more steps than a tile keeps in flight, uneven
   ones, one range and as many as steps, partial tiles in M and N.
-* fp32 SwiGLU at both tile sizes, against 64 bits.
+* fp32 SwiGLU at every tile size, against 64 bits.
 """
 from __future__ import annotations
 
@@ -58,7 +58,7 @@ def test_partial_sums_of_every_range(lib, rows, steps, ranges):  # noqa: F811
         assert bool(got[ranges].isnan().all()), "written past the last range"
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (17, 33, 68), (66, 688, 256), (31, 47, 100), (1030, 1041, 33), (2032, 688, 256)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (17, 33, 68), (66, 688, 256), (31, 47, 100), (1030, 1041, 33), (2032, 688, 256), (2048, 2048, 36), (1985, 2047, 12)])
 def test_fp32_swiglu_against_64_bits(lib, M, N, K):  # noqa: F811
     """Gate and up are within e = (K + 2) 2^-24 sum |a| |w| of the product each (K
     products, K + 1 sums); |silu'| < 1.1; and silu * up, an exponential, a sum, a
