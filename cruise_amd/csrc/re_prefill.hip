@@ -631,10 +631,11 @@ __global__ void __launch_bounds__(kGthreads, 1) k_gemm_bf16(GemmArgs a, int nM, 
 // products.  Bound by the vector units' rate and LDS reads, 70-77 TFLOP/s;
 // the matrix-core kernel below reads its operands from L2 for every 32 x 32 tile
 // and stays at 60 (22-27 where it has to load element by element).  See
-// gemm_f32_launch.  m_on_x: the grid's first dimension runs over M tiles, else
-// over N tiles.
+// gemm_f32_launch.  Eight workgroups per CU (64 registers): at seven, 3,424 x
+// 2,235 x 1,348 takes 352 us instead of 333.  m_on_x: the grid's first dimension
+// runs over M tiles, else over N tiles.
 template <int EPI>
-__global__ void __launch_bounds__(256) k_gemm_f32_lds(GemmArgs a, int m_on_x) {
+__global__ void __launch_bounds__(256, 8) k_gemm_f32_lds(GemmArgs a, int m_on_x) {
   constexpr bool kSwiGlu = EPI == kGemmSwiGlu;
   constexpr int kTileN = kSwiGlu ? 32 : 64;
   __shared__ float As[16][64 + 4];
@@ -1287,10 +1288,11 @@ static hipError_t gemm_launch_mj(const GemmArgs& a, const GemmPlan& p, hipStream
 }
 
 // Three kernels by the number of tiles, so that each still gives every CU work:
-// - through LDS from four tiles per CU on, where both operands can be read 16
-//   bytes at a time, else past one per CU.  Matrix cores and LDS (M x N x K):
-//   1,000 x 3,584 x 1,024 (896 tiles) 140 and 147 us, 2,000 x 2,048 x 1,024
-//   (1,024) 155 and 149, 4,096 x 4,096 x 1,024 (4,096) 597 and 487; 4-byte
+// - through LDS from three tiles per CU on (SwiGLU: four), where both operands
+//   can be read 16 bytes at a time, else past one per CU.  Matrix cores and LDS
+//   (M x N x K): 1,000 x 2,048 x 1,024 (512 tiles) 88 and 97 us, 1,000 x 3,584 x
+//   1,024 (896) 142 and 142, 16,000 x 256 x 688 (1,000) 116 and 102, 2,000 x
+//   2,048 x 1,024 (1,024) 157 and 145, 4,096 x 4,096 x 1,024 596 and 479; 4-byte
 //   loads, 1,000 x 1,000 x 1,023 (256) 95 and 110, 1,024 x 1,536 x 1,023 (384)
 //   143 and 109, 4,096 x 4,096 x 1,023 1,413 and 503.  SwiGLU: 512 x 3,584 x
 //   1,024 (896) 136 and 142, 1,000 x 2,048 x 1,024 (1,024) 148 and 146, 4,096 x
@@ -1310,7 +1312,7 @@ static hipError_t gemm_f32_launch(const GemmArgs& a, hipStream_t stream) {
   constexpr unsigned kTileN = EPI == kGemmSwiGlu ? 32 : 64;
   const unsigned m_tiles = (a.M + 63u) / 64, n_tiles = (a.N + kTileN - 1) / kTileN;
   const unsigned long long lds_tiles = (unsigned long long)m_tiles * n_tiles;
-  if (vec ? lds_tiles >= 4 * kCus : lds_tiles > kCus) {
+  if (vec ? lds_tiles >= (EPI == kGemmSwiGlu ? 4 : 3) * kCus : lds_tiles > kCus) {
     // N tiles next to each other share A's rows in L2; a grid's second dimension holds 65,535
     const int m_on_x = m_tiles > 65535;
     k_gemm_f32_lds<EPI><<<m_on_x ? dim3(m_tiles, n_tiles) : dim3(n_tiles, m_tiles), 256, 0, stream>>>(a, m_on_x);

@@ -2,7 +2,7 @@
 split over four waves, and 64 x 64 tiles through LDS for large products.
 
 * Edges of the tiles, of the 16-element K chunks and of the four waves' turns,
-  every tile size (32 x 32 from 512 tiles on; 64 x 64 from 1,024 on, unaligned
+  every tile size (32 x 32 from 512 tiles on; 64 x 64 from 768 on, unaligned
   from 257 on), aligned and unaligned rows, against the product in 64 bits.  Each output is K products and K + 2 sums in
   fp32 (the bias or residual one of them), so it is within
   (K + 3) 2^-24 (sum |a| |w| + |bias or residual|) of it in any order.
@@ -30,7 +30,7 @@ pytestmark = pytest.mark.gpu
 
 SMALL = [(1, 1, 1), (15, 17, 3), (16, 16, 64), (17, 33, 68), (66, 256, 688), (31, 48, 272), (5, 7, 1000)]
 LARGE = [(512, 1024, 16), (496, 1024, 40), (1030, 1041, 33), (2032, 688, 256), (1024, 1024, 20), (1025, 1024, 7),
-         (2048, 2048, 36), (1985, 2047, 12), (1984, 2112, 64)]
+         (2048, 1472, 36), (2048, 1536, 36), (2048, 2048, 36), (1985, 2047, 12), (1984, 2112, 64)]
 
 
 @pytest.mark.parametrize("M,N,K", SMALL + LARGE)
